@@ -85,9 +85,19 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
         bad_l |= n < 0;
         if (n > 0) R_l = max(R_l, r);
     }
-    const bool qbad = P.qinfo[row * 5 + 4] != 0;
-    int flag = (__ballot(bad_l) != 0 || qbad) ? 1 : 0;
     const int R = wave_max_i(R_l);
+    // a NaN/inf in q flags the row. Partials with keys carry that flag already when the multi-row
+    // kernel wrote them (no score of such a row is finite); a row without keys is looked at here
+    bool qbad = false;
+    if (!P.mrow) {
+        qbad = P.qinfo[row * 5 + 4] != 0;
+    } else if (R == INT_MIN) {
+        const uint16_t* qr = P.q + b * P.g.q_seq_stride + (int64_t)t * P.g.q_tok_stride + (int64_t)hq * P.g.q_head_stride;
+        bool nf = false;
+        for (int i = lane; i < P.g.head_dim; i += 64) nf |= ((qr[i] >> 7) & 0xFF) == 0xFF;
+        qbad = __ballot(nf) != 0;
+    }
+    int flag = (__ballot(bad_l) != 0 || qbad) ? 1 : 0;
     uint16_t* o16 = (uint16_t*)P.out;
     uint32_t* o32 = (uint32_t*)P.out;
     const int64_t obase = b * P.g.o_seq_stride + (int64_t)t * P.g.o_tok_stride + (int64_t)hq * P.g.o_head_stride;

@@ -3,7 +3,8 @@
 // One step is four launches on the caller's stream, with fixed grids and no memsets:
 //   ea_prep      q rows -> fp64 + exponent ranges; clears the tier-2 work counter (the decode
 //                kernel on uniform splits does both itself, and the step is three launches)
-//   ea_split     tier 1: per (segment, row block, KV split) an fp64 pass over 64-key tiles:
+//   ea_split     tier 1 (ea_decode, ea_mrow where they apply): per (segment, row block, KV split) an
+//                fp64 pass over 64-key tiles:
 //                exact scores (checked), certified logits and weights, P.V partials with
 //                rigorous error bounds. Writes one partial per (split, row).
 //   ea_combine   merges the split partials in the caller's order and certifies RN(N/Z) per
@@ -34,36 +35,41 @@ using namespace ea;
 // one wave per row; block 0 clears the tier-2 work list, and on the decode kernel's stream plan an
 // extra last block writes that plan.
 // ------------------------------------------------------------------------------------------------
-// The decode kernel's equal-share plan (Params::dq_*), by one 256-thread block: per unit its tile
+// The decode kernel's equal-share plan (Params::dq_*), by one block of NT threads: per unit its tile
 // count (up to unit_kend, at most dq_max_tiles), the exclusive prefix sums S_u with S_units = W, the
 // share max(ceil(W / dq_blocks), dq_min_share), and per block g its first piece as one record
 // (unit u, S_u, S_(u+1), share): the unit holding tile g share is the u with
 // S_u <= g share < S_(u+1), so the blocks g in [ceil(S_u / share), ceil(S_(u+1) / share)) start in
 // unit u and each is written by that unit's thread. Blocks past W get u = units. Every entry the
 // decode kernel and the combine read is written here.
+template <int NT>
 __device__ void dq_plan_block(const Params& P) {
-    __shared__ int s_scan[2][256];
+    __shared__ int s_scan[2][NT];
     __shared__ int s_share;
     const int tid = threadIdx.x, U = P.dq_units, G = P.dq_blocks;
     int32_t* plan = P.dq_plan;
     int32_t* Su = plan + 2;
     int4* brec = (int4*)(plan + P.dq_rec_off);
-    const int per = (U + 255) / 256;
+    const int per = (U + NT - 1) / NT;
     const int u0 = min(tid * per, U), u1 = min(u0 + per, U);
-    auto tiles = [&](int u) { return min((unit_kend(P, u / P.nrb, u % P.nrb) + 63) >> 6, P.dq_max_tiles); };
+    // each thread's units twice: their tile counts, kept in Su, and then the prefix sums over them
     int sum = 0;
-    for (int u = u0; u < u1; ++u) sum += tiles(u);
-    // inclusive scan of the 256 chunk sums (Hillis-Steele, ping-pong)
+    for (int u = u0; u < u1; ++u) {
+        const int t = min((unit_kend(P, u / P.nrb, u % P.nrb) + 63) >> 6, P.dq_max_tiles);
+        Su[u] = t;
+        sum += t;
+    }
+    // inclusive scan of the chunk sums (Hillis-Steele, ping-pong)
     int cur = 0;
     s_scan[0][tid] = sum;
     __syncthreads();
-    for (int o = 1; o < 256; o <<= 1) {
+    for (int o = 1; o < NT; o <<= 1) {
         const int x = s_scan[cur][tid] + (tid >= o ? s_scan[cur][tid - o] : 0);
         s_scan[cur ^ 1][tid] = x;
         cur ^= 1;
         __syncthreads();
     }
-    const int W = s_scan[cur][255];
+    const int W = s_scan[cur][NT - 1];
     if (tid == 0) {
         const int share = max(max((W + G - 1) / G, P.dq_min_share), 1);
         s_share = share;
@@ -76,20 +82,26 @@ __device__ void dq_plan_block(const Params& P) {
     const int share = s_share;
     int run = s_scan[cur][tid] - sum;  // exclusive prefix of this thread's chunk
     for (int u = u0; u < u1; ++u) {
-        const int t = tiles(u);
+        const int t = Su[u];
         Su[u] = run;
         for (int g = (run + share - 1) / share; g * share < run + t && g < G; ++g)
             brec[g] = make_int4(u, run, run + t, share);
         run += t;
     }
     const int nb = (W + share - 1) / share;  // blocks with a share: [0, nb)
-    for (int g = nb + tid; g < G; g += 256) brec[g] = make_int4(U, W, W, share);
+    for (int g = nb + tid; g < G; g += NT) brec[g] = make_int4(U, W, W, share);
+}
+
+// The equal-share plan alone (the multi-row kernel's steps), and the cleared tier-2 work list.
+__global__ void __launch_bounds__(1024) ea_plan(Params P) {
+    if (threadIdx.x <= EA_T2_BLOCKS) P.wl_cnt[threadIdx.x] = 0;
+    dq_plan_block<1024>(P);
 }
 
 __global__ void __launch_bounds__(256) ea_prep(Params P) {
     if (blockIdx.x == 0 && threadIdx.x <= EA_T2_BLOCKS) P.wl_cnt[threadIdx.x] = 0;
     if (P.dq_stream && blockIdx.x == gridDim.x - 1) {
-        dq_plan_block(P);  // the extra last block
+        dq_plan_block<256>(P);  // the extra last block
         return;
     }
     int lane = threadIdx.x & 63;
@@ -1233,15 +1245,80 @@ struct Plan {
     int t2_keys;
     int prefill, pf_ntiles, pf_nrb, pf_nsplit, pf_tps;
     // the decode kernel's equal-share decomposition (Params::dq_*): dq = 1 when the geometry may
-    // take it (the pointer checks come at launch); nsplit_gen = the general kernel's uniform split
-    // count, nsplit = nsplit_gen + 1 partial slots per unit for the decode kernel's pieces
-    int dq, nsplit_gen, dq_units, dq_min_share, dq_max_tiles, dq_rec_off;
+    // take it (the pointer checks come at launch); nsplit_gen = the uniform split count, nsplit =
+    // the partial slots per unit (one more for the pieces of the equal-share plan)
+    int dq, nsplit_gen, dq_units, dq_max_tiles, dq_rec_off;
+    // the multi-row kernel (ea_mrow.hip): its rows per block (0: not taken). Its row blocks per
+    // segment are rb and nrb, its splits nsplit_gen and split_len; gen_* are those of the kernel that
+    // runs when the pointers do not suit it (the same values where it is not taken)
+    int mrow, gen_rb, gen_nrb, gen_nsplit, gen_split_len;
 };
 
 // most blocks the decode kernel's equal-share decomposition launches (the plan array's size)
 #define EA_DQ_MAX_BLOCKS 4096
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Rows per block of the multi-row kernel for this geometry, 0 where another kernel takes the step.
+// d = dv = 128: from 3 rows per segment on (1 and 2 rows are what ea_decode's 2-row blocks are for:
+// 32 x 4K keys 108 us there) up to where the int8 prefill kernel starts. Any other head size: always
+// (ea_split takes what the pointers or pages do not allow).
+int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {
+    if (o->timers || o->kernel == EA_KERNEL_GENERAL) return 0;
+    if (g->head_dim == 128 && g->head_dim_v == 128) {
+        int nt = 0, nr = 0;
+        if (r_seg <= 2 || ea_prefill_eligible(*g, g->num_q_heads / g->num_kv_heads, o->kernel, &nt, &nr)) return 0;
+    }
+    return r_seg <= 4 ? 4 : (r_seg <= 8 ? 8 : 16);
+}
+
+// ns splits of maxlen keys in whole tiles
+void split_tiles(int maxlen, int ns, int* nsplit, int* split_len) {
+    int sl = (maxlen + ns - 1) / ns;
+    sl = (sl + EA_TILE - 1) / EA_TILE * EA_TILE;
+    if (sl < EA_TILE) sl = EA_TILE;
+    *split_len = sl;
+    *nsplit = std::max(1, (maxlen + sl - 1) / sl);
+}
+
+// KV splits of a step of `items` (segment, row block) units: the caller's count or one for the
+// device, in whole tiles.
+void choose_splits(int64_t items, int maxlen, int splits, int* nsplit, int* split_len) {
+    int ns = splits;
+    if (ns == 0) {
+        // enough work items for 256 CUs x 2 blocks, splits of at least 256 keys
+        ns = 1;
+        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 256) ns *= 2;
+        // and splits of at most 2048 keys: with sequence lengths that differ (only their maximum
+        // is known here), long splits leave the blocks of short sequences idle while the longest
+        // block runs, and the last round of blocks is sparse (C5, 8K-131K keys: 8 splits 1.36 ms,
+        // 32 splits 1.19-1.21 ms, 63 splits 1.16-1.19 ms per step)
+        while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
+    }
+    split_tiles(maxlen, ns, nsplit, split_len);
+}
+
+// The same for the multi-row kernel. First enough blocks to fill the device, down to one tile per
+// split: a short context then takes a step or two per wave instead of a chain of them. Then splits
+// of at most 512 keys, so that the equal-share plan (taken past one round of resident blocks) can
+// even out sequences of different lengths in shares of 8 tiles, while the partials stay below
+// MROW_PART and the workspace below the allocation-free entry point's array.
+void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsplit, int* split_len) {
+    int ns = splits;
+    if (ns == 0) {
+        const int64_t MROW_PART = 32 << 20, MROW_WS = 96 << 20;
+        const int64_t units = (int64_t)pl.nseg * pl.nrb;
+        const int64_t items = pl.r_seg <= 8 ? (int64_t)pl.nseg * ((pl.r_seg + 1) / 2) : 2 * units;
+        const int64_t rest = (int64_t)EA_T2_BLOCKS * 12 * maxlen + pl.rows * 1100;
+        ns = 1;
+        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 64) ns *= 2;
+        while ((int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART &&
+               2 * ns * pl.rows * dv * 8 + rest <= MROW_WS)
+            ns *= 2;
+        while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
+    }
+    split_tiles(maxlen, ns, nsplit, split_len);
+}
 
 int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     if (!g || !o) return -1;
@@ -1263,6 +1340,13 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     const bool dec_rows = g->head_dim == 128 && g->head_dim_v == 128 && o->kernel != EA_KERNEL_GENERAL && !o->timers;
     pl->rb = dec_rows ? std::min(pl->r_seg, 2) : (pl->r_seg >= 3 ? 4 : pl->r_seg);
     pl->nrb = (pl->r_seg + pl->rb - 1) / pl->rb;
+    pl->gen_rb = pl->rb;
+    pl->gen_nrb = pl->nrb;
+    pl->mrow = mrow_rows(g, o, pl->r_seg);
+    if (pl->mrow) {
+        pl->rb = pl->mrow;
+        pl->nrb = (pl->r_seg + pl->rb - 1) / pl->rb;
+    }
     pl->nseg = g->num_seqs * g->num_kv_heads;
     pl->rows = (int64_t)g->num_seqs * g->num_tokens * g->num_q_heads;
     int ps = 0;
@@ -1272,38 +1356,25 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     while ((1 << dl) < g->head_dim) ++dl;
     pl->dlog = dl;
     int maxlen = g->max_seq_len > 0 ? g->max_seq_len : 1;
-    int ns = o->splits;
-    if (ns == 0) {
-        // enough work items for 256 CUs x 2 blocks, splits of at least 256 keys
-        int64_t items = (int64_t)pl->nseg * pl->nrb;
-        ns = 1;
-        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 256) ns *= 2;
-        // and splits of at most 2048 keys: with sequence lengths that differ (only their maximum
-        // is known here), long splits leave the blocks of short sequences idle while the longest
-        // block runs, and the last round of blocks is sparse (C5, 8K-131K keys: 8 splits 1.36 ms,
-        // 32 splits 1.19-1.21 ms, 63 splits 1.16-1.19 ms per step)
-        while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
-    }
-    int sl = (maxlen + ns - 1) / ns;
-    sl = (sl + EA_TILE - 1) / EA_TILE * EA_TILE;
-    if (sl < EA_TILE) sl = EA_TILE;
-    pl->split_len = sl;
-    pl->nsplit = (maxlen + sl - 1) / sl;
-    if (pl->nsplit < 1) pl->nsplit = 1;
-    pl->nsplit_gen = pl->nsplit;
+    choose_splits(pl->nseg * (int64_t)pl->gen_nrb, maxlen, o->splits, &pl->gen_nsplit, &pl->gen_split_len);
+    pl->nsplit_gen = pl->gen_nsplit;
+    pl->split_len = pl->gen_split_len;
+    if (pl->mrow) choose_splits_mrow(*pl, maxlen, g->head_dim_v, o->splits, &pl->nsplit_gen, &pl->split_len);
+    // partial slots per unit, for whichever of the two kernels the pointers allow
+    pl->nsplit = std::max(pl->nsplit_gen, pl->gen_nsplit);
     // the d = 128 decode kernel may run this step (ea_launch_decode also checks the pointers):
     // its pieces need nsplit + 1 partial slots per unit
     const int64_t max_tiles = ((int64_t)maxlen + 63) / 64;
+    const int64_t max_nrb = std::max(pl->nrb, pl->gen_nrb);
     int pf_nt = 0, pf_nr = 0;
-    pl->dq = g->head_dim == 128 && g->head_dim_v == 128 && o->kernel != EA_KERNEL_GENERAL && !o->timers &&
-             !ea_prefill_eligible(*g, pl->grp, o->kernel, &pf_nt, &pf_nr) && pl->rows < ((int64_t)1 << 30) &&
+    pl->dq = (pl->mrow || (g->head_dim == 128 && g->head_dim_v == 128)) && o->kernel != EA_KERNEL_GENERAL &&
+             !o->timers && !ea_prefill_eligible(*g, pl->grp, o->kernel, &pf_nt, &pf_nr) && pl->rows < ((int64_t)1 << 30) &&
              (int64_t)maxlen + 64 < ((int64_t)1 << 30) &&
-             (int64_t)pl->nseg * pl->nrb * max_tiles < ((int64_t)1 << 30) &&
-             (int64_t)pl->nseg * pl->nrb < ((int64_t)1 << 24);
-    pl->dq_units = pl->nseg * pl->nrb;
+             (int64_t)pl->nseg * max_nrb * max_tiles < ((int64_t)1 << 30) &&
+             (int64_t)pl->nseg * max_nrb < ((int64_t)1 << 24);
+    pl->dq_units = (int)std::min<int64_t>(pl->nseg * max_nrb, 1 << 24);
     pl->dq_max_tiles = (int)max_tiles;
-    pl->dq_min_share = (int)((max_tiles + pl->nsplit_gen - 1) / pl->nsplit_gen);
-    if (pl->dq) pl->nsplit = pl->nsplit_gen + 1;
+    if (pl->dq) ++pl->nsplit;
     int64_t R = pl->rows;
     int dv = g->head_dim_v;
     size_t off = 0;
@@ -1314,7 +1385,7 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     pl->off_pn = off; off = align_up(off + (size_t)pl->nsplit * R * 4);
     pl->off_pZ = off; off = align_up(off + (size_t)pl->nsplit * R * 8);
     pl->off_pN = off; off = align_up(off + (size_t)pl->nsplit * R * dv * 8);
-    pl->off_pV = off; off = align_up(off + (size_t)pl->nsplit * pl->nseg * pl->nrb * dv * 4);
+    pl->off_pV = off; off = align_up(off + (size_t)pl->nsplit * pl->nseg * std::max(pl->nrb, pl->gen_nrb) * dv * 4);
     pl->off_wl = off; off = align_up(off + (size_t)(R > 0 ? R : 1) * 4);
     pl->off_cnt = off; off = align_up(off + 4 * (1 + EA_T2_BLOCKS));
     pl->off_t2part = off; off = align_up(off + EA_T2_BLOCKS * sizeof(T2Part));
@@ -1495,29 +1566,39 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     P.dq_stream = 0;
     bool use_decode = false;
     if (!pl.prefill) {
-        P.nsplit = pl.nsplit_gen;
-        use_decode = pl.dq && pl.nseg > 0 && ea_decode_eligible(P);
-        int slots = 0, cus = 0;
+        int slots = 0, cus = 0, nsplit = pl.nsplit_gen;
+        if (pl.mrow && pl.nseg > 0 && ea_mrow_eligible(P)) {
+            P.mrow = 1;
+            if ((rc = ea_mrow_slots(P, &slots))) return rc;
+        } else if (pl.mrow) {
+            P.rb = pl.gen_rb;
+            P.nrb = pl.gen_nrb;
+            P.split_len = pl.gen_split_len;
+            nsplit = pl.gen_nsplit;
+        }
+        P.nsplit = nsplit;
+        use_decode = !P.mrow && pl.dq && pl.nseg > 0 && ea_decode_eligible(P);
         if (use_decode && (rc = ea_decode_slots(P, &slots, &cus))) return rc;
+        const int64_t units = (int64_t)P.nseg * P.nrb;
         // the equal-share plan when the uniform split grid would take more than one round of
         // resident blocks (long or ragged contexts); otherwise one block per (unit, split)
         P.dq_lead = 0;
-        if (use_decode) P.pv_tiles = pl.split_len / EA_TILE;
-        if (use_decode && pl.nsplit_gen >= 2 && (int64_t)pl.dq_units * pl.nsplit_gen == slots && slots > cus) {
+        if (use_decode || P.mrow) P.pv_tiles = P.split_len / EA_TILE;
+        if (use_decode && nsplit >= 2 && units * nsplit == slots && slots > cus) {
             // exactly one round: the first wave's splits are weighted 5 against 4 (the decode
             // kernel's uniform path); the longest is at most 5 / (5 + 4 (n - 1)) of the unit's
             // tiles, plus one for the rounding
-            const int64_t tt = (int64_t)pl.nsplit_gen * (pl.split_len / EA_TILE), den = 5 + 4 * (int64_t)(pl.nsplit_gen - 1);
+            const int64_t tt = (int64_t)nsplit * (P.split_len / EA_TILE), den = 5 + 4 * (int64_t)(nsplit - 1);
             P.dq_lead = cus;
             P.pv_tiles = (int32_t)((5 * tt + den - 1) / den + 1);
         }
-        if (use_decode && (int64_t)pl.dq_units * pl.nsplit_gen > slots) {
+        if ((use_decode || (P.mrow && pl.dq)) && units * nsplit > slots) {
             const int64_t nb = std::min<int64_t>(slots, EA_DQ_MAX_BLOCKS);
             P.dq_stream = 1;
-            P.nsplit = pl.nsplit;
-            P.dq_units = pl.dq_units;
+            P.nsplit = nsplit + 1;
+            P.dq_units = (int32_t)units;
             P.dq_blocks = (int32_t)(nb > 0 ? nb : 1);
-            P.dq_min_share = pl.dq_min_share;
+            P.dq_min_share = (pl.dq_max_tiles + nsplit - 1) / nsplit;
             P.dq_max_tiles = pl.dq_max_tiles;
             P.dq_rec_off = pl.dq_rec_off;
             P.dq_plan = (int32_t*)(ws + pl.off_dq);
@@ -1545,7 +1626,13 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         return mark(4);
     }
     // the decode kernel on uniform splits prepares its own rows' q (and clears the work list)
-    if (!(use_decode && !P.dq_stream)) {
+    if (P.mrow) {
+        // the multi-row kernel converts its own q rows; the plan is one block's work
+        if (P.dq_stream) {
+            hipLaunchKernelGGL(ea_plan, dim3(1), dim3(1024), 0, st, P);
+            if ((rc = herr(hipGetLastError()))) return rc;
+        }
+    } else if (!(use_decode && !P.dq_stream)) {
         hipLaunchKernelGGL(ea_prep, dim3(rb4 + (P.dq_stream ? 1u : 0u)), dim3(256), 0, st, P);
         rc = herr(hipGetLastError());
         if (rc) return rc;
@@ -1565,19 +1652,21 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         });
         rc = herr(attr_err);
         if (rc) return rc;
-        dim3 grid((unsigned)(pl.nseg * pl.nrb), (unsigned)pl.nsplit_gen);
+        dim3 grid((unsigned)(P.nseg * P.nrb), (unsigned)P.nsplit);
         if ((rc = mark(1))) return rc;
         const dim3 blk(EA_THREADS);
         const size_t lds = sizeof(SplitSmem);
-        if (use_decode) {
+        if (P.mrow) {
+            if ((rc = ea_launch_mrow(P, st))) return rc;
+        } else if (use_decode) {
             if ((rc = ea_launch_decode(P, st))) return rc;
         } else if (o->timers) {
-            if (pl.rb == 1) hipLaunchKernelGGL((ea_split<1, true>), grid, blk, lds, st, P);
-            else if (pl.rb == 2) hipLaunchKernelGGL((ea_split<2, true>), grid, blk, lds, st, P);
+            if (P.rb == 1) hipLaunchKernelGGL((ea_split<1, true>), grid, blk, lds, st, P);
+            else if (P.rb == 2) hipLaunchKernelGGL((ea_split<2, true>), grid, blk, lds, st, P);
             else hipLaunchKernelGGL((ea_split<4, true>), grid, blk, lds, st, P);
         } else {
-            if (pl.rb == 1) hipLaunchKernelGGL((ea_split<1, false>), grid, blk, lds, st, P);
-            else if (pl.rb == 2) hipLaunchKernelGGL((ea_split<2, false>), grid, blk, lds, st, P);
+            if (P.rb == 1) hipLaunchKernelGGL((ea_split<1, false>), grid, blk, lds, st, P);
+            else if (P.rb == 2) hipLaunchKernelGGL((ea_split<2, false>), grid, blk, lds, st, P);
             else hipLaunchKernelGGL((ea_split<4, false>), grid, blk, lds, st, P);
         }
         rc = herr(hipGetLastError());

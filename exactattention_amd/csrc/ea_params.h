@@ -101,6 +101,9 @@ struct Params {
     // [0, nsplit split_len) is cut in whole tiles in proportion to weights 5 for its splits among
     // them and 4 for the others. 0: equal splits of split_len.
     int32_t dq_lead;
+    // 1: the multi-row split kernel wrote the partials (it keeps no qinfo: the combine looks at the
+    // q row itself where a row has no visible key)
+    int32_t mrow;
 };
 
 __device__ __forceinline__ int64_t row_index(const Params& P, int64_t b, int t, int hq) {
@@ -117,8 +120,9 @@ __device__ inline int unit_kend(const Params& P, int seg, int rbk) {
     const int nrow = min(P.rb, P.r_seg - row0);
     const int tb = P.tree_mask ? P.tree_base[b] : 0;
     int kend = 0;
-    for (int r = 0; r < nrow; ++r) {
-        const int t = (row0 + r) / P.grp;
+    // the block's rows are query heads of consecutive tokens
+    const int t1 = (row0 + nrow - 1) / P.grp;
+    for (int t = row0 / P.grp; t <= t1; ++t) {
         const int64_t tok = (int64_t)b * P.g.num_tokens + t;
         int e = P.kv_len[tok];
         const uint64_t m = P.tree_mask ? P.tree_mask[tok] : 0ull;
@@ -230,6 +234,11 @@ __device__ __forceinline__ int wave_sum_i(int x) {
 int ea_decode_eligible(const Params& P);
 int ea_decode_slots(const Params& P, int* slots, int* cus = nullptr);
 int ea_launch_decode(const Params& P, hipStream_t st);
+// The multi-row split kernel (ea_mrow.hip): row blocks of P.rb = 4, 8 or 16, any head sizes. The
+// same three questions as for the decode kernel.
+int ea_mrow_eligible(const Params& P);
+int ea_mrow_slots(const Params& P, int* slots);
+int ea_launch_mrow(const Params& P, hipStream_t st);
 
 // int8-MFMA prefill path (ea_prefill.hip). A tile holds 64 keys of one segment:
 //   [0, 32768)       K digit planes t = 0..3: [t][key 64][128 bytes], 16-byte chunk c of key k

@@ -161,7 +161,7 @@ __device__ __forceinline__ int3 pf_cold_pair(int mode, const uint8_t* qrow, int 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Branch-free certified t = RN32(alpha s) and w = RN24(2^t) = M 2^E for 4 pairs in lock step
+// Branch-free certified t = RN32(alpha s) and w = RN24(2^t) = M 2^E for NP pairs in lock step
 // (independent chains the scheduler interleaves). xs: fp64 scores in units 2^lsbq; a = alpha 2^lsbq;
 // adel >= (1 + 2^-50) |a| |xs - exact| (the score bound with its rounding slack). p + pe = a xs
 // exactly (FMA). The interval around p + pe rounds to t0 = RN32(p) when |p + pe - t0| + adel is
@@ -173,13 +173,14 @@ __device__ __forceinline__ int3 pf_cold_pair(int mode, const uint8_t* qrow, int 
 // subtracting 1.5 * 2^52; certified when |Y - RN(Y)| <= 1/2 - 2^-26 (the fp64 evaluation error
 // is below 2^-26.9). ok[i] false: the exact path decides.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void cert4(const double (&xs)[4], const double (&adel)[4], double a, const double* T1s,
-                                      const double* T2, int (&M)[4], int (&E)[4], bool (&ok)[4]) {
+template <int NP>
+__device__ __forceinline__ void cert_pairs(const double (&xs)[NP], const double (&adel)[NP], double a, const double* T1s,
+                                           const double* T2, int (&M)[NP], int (&E)[NP], bool (&ok)[NP]) {
     const double c1 = u64_as_f64(EA_C_BITS[0]) * 0x1p-16, c2 = u64_as_f64(EA_C_BITS[1]) * 0x1p-32,
                  c3 = u64_as_f64(EA_C_BITS[2]) * 0x1p-48;
-    double d0[4];
+    double d0[NP];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NP; ++i) {
         const double p = a * xs[i];
         const double pe = __fma_rn(a, xs[i], -p);
         const float tf = (float)p;
@@ -195,21 +196,21 @@ __device__ __forceinline__ void cert4(const double (&xs)[4], const double (&adel
         ok[i] = tiny | inner;
         d0[i] = tiny ? 0.0 : t0;
     }
-    double fl[4], rr[4];
-    int idx[4];
+    double fl[NP], rr[NP];
+    int idx[NP];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NP; ++i) {
         fl[i] = floor(d0[i]);
         const double t16 = (d0[i] - fl[i]) * 65536.0;  // exact: d0 is an fp32 value below 2^30
         const double fi = floor(t16);
         idx[i] = (int)fi;
         rr[i] = t16 - fi;
     }
-    double aa[4];
+    double aa[NP];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) aa[i] = T1s[idx[i] >> 8] * T2[idx[i] & 255];
+    for (int i = 0; i < NP; ++i) aa[i] = T1s[idx[i] >> 8] * T2[idx[i] & 255];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NP; ++i) {
         const double poly = rr[i] * __fma_rn(rr[i], __fma_rn(rr[i], c3, c2), c1);
         const double Y = __fma_rn(aa[i], poly, aa[i]);
         const double Yr = (Y + 0x1.8p52) - 0x1.8p52;

@@ -860,7 +860,7 @@ __global__ void __launch_bounds__(64 * NWB, 1) ea_pf_main(Params P) {
             pv_mfma(Wd, sVp, kk * (NCT / NKT), (kk + 1) * (NCT / NKT));
             int M[4], E[4];
             bool ok[4];
-            cert4(xs[kk], adel[kk], qm.a, T1s, T2, M, E, ok);
+            cert_pairs<4>(xs[kk], adel[kk], qm.a, T1s, T2, M, E, ok);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const bool vis = (vism >> (4 * kk + i)) & 1;

@@ -91,13 +91,14 @@ typedef struct ea_options {
                                certified, [6] tier-1 weights not certified, [7] tier-1 final
                                roundings not certified, [8] scores taken by the per-pair exact
                                path, [9] rows whose tier 1 ran in the d = 128 decode
-                               kernel, [10] rows whose tier 1 ran in the int8-MFMA
+                               kernel or the multi-row kernel (3 to 31 rows per
+                               sequence and KV head, and head sizes other than 128), [10] rows whose tier 1 ran in the int8-MFMA
                                prefill kernel, [11] prefill epoch folds before the last
                                tile (waves), [12] prefill waves that ran the exact
                                per-pair path, [13] rows certified by the host exact
                                tier (ea_hip_exact_rows), [14] rows it refused (spread
                                limit, flag 2), [15] steps whose decode kernel ran
-                               the equal-share plan */
+                               the equal-share plan (either kernel) */
     void* const* events;    /* optional: 5 hipEvent_t recorded on `stream` before prep (the
                                int8 path: q and K/V slicing; none on the decode kernel's uniform
                                grid, whose kernel converts q), the tier-1 kernel, the combine (the

@@ -1,0 +1,117 @@
+"""The multi-row split kernel (ea_mrow.hip) at the edges of its row blocks (4, 8, 16 rows), key steps
+(16 keys per wave, 64 per tile), splits and head sizes, against the oracle. Every result is
+certified, so the bar is equal bits."""
+
+import numpy as np
+import pytest
+
+from exactattention_amd import problem
+from exactattention_amd.formats import default_alpha_bits
+from gen import bf16
+from test_gpu_parity import _oracle, _rand_problem, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(prob, ab, out="bf16", splits=0):
+    want, wflags = _oracle(prob, ab, out)
+    got, flags, st = _run(prob, ab, out, splits)
+    assert st["decode_kernel_rows"] == flags.size, st
+    assert not flags.any() and not np.any(wflags), st
+    assert np.array_equal(got, want), st
+    return st
+
+
+@pytest.mark.parametrize("T,grp", [(1, 3), (1, 4), (5, 1), (2, 4), (3, 3), (1, 16), (17, 1), (9, 2)])
+@pytest.mark.parametrize("d,dv", [(8, 4), (64, 64), (72, 40), (128, 64), (96, 96), (128, 128)])
+def test_rows_and_head_sizes(gpu, T, grp, d, dv):
+    """3 to 18 rows per segment (one full row block, one row more, a partial one), head sizes on both
+    sides of the 64-dim variant and with dims or channels that fill a chunk only in part; one key,
+    a wave's step and a tile with one key less and more, and several splits. Contiguous and paged."""
+    rng = np.random.default_rng(1000 * T + 100 * grp + d + dv)
+    ab = default_alpha_bits(d)
+    for S, page in ((T, 0), (15 + T, 16), (16, 0), (17, 64), (63 + T, 0), (64, 16), (65 + T, 16), (777, 64)):
+        prob = _rand_problem(rng, "normal", "normal", B=2, T=T, Hq=2 * grp, Hkv=2, S=max(S, T), d=d, dv=dv)
+        if page:
+            prob = problem.to_paged(prob, page, rng, "HND" if S & 1 else "NHD")
+        _check(prob, ab, "fp32" if S & 2 else "bf16", splits=3 if S == 777 else 0)
+
+
+@pytest.mark.parametrize("rows", [4, 8, 16])
+@pytest.mark.parametrize("kind", ["wide", "outlier", "dupes", "subnormal"])
+def test_value_kinds(gpu, rows, kind):
+    """Scores that cancel over 48 binades, exact zeros and ties, subnormals; and logits hundreds apart
+    (alpha 8), so that reference exponents move by more than their headroom."""
+    rng = np.random.default_rng(rows)
+    for d, alpha in ((128, None), (64, np.float32(8.0))):
+        prob = _rand_problem(rng, kind, kind, B=2, T=1, Hq=2 * rows, Hkv=2, S=1500, d=d, dv=d)
+        ab = default_alpha_bits(d) if alpha is None else int(alpha.view(np.uint32))
+        want, wflags = _oracle(prob, ab)
+        got, flags, st = _run(prob, ab)
+        assert st["decode_kernel_rows"] == flags.size, st
+        ok = flags.reshape(want.shape[:3]) == 0  # what the device tiers leave is the host tier's
+        assert np.array_equal(got[ok], want[ok]) and (flags != 2).all(), st
+
+
+@pytest.mark.parametrize("rows", [4, 8, 16])
+def test_every_pair_waits(gpu, rows):
+    """Logits exactly half way between two fp32 values for every pair (alpha 1, s = k0 + 2^-24 with k0
+    in [1, 2), in the even rows): no interval decides them, so every step fills the wave's list."""
+    rng = np.random.default_rng(rows)
+    prob = _rand_problem(rng, "normal", "normal", B=2, T=1, Hq=2 * rows, Hkv=2, S=1000, d=64, dv=64)
+    prob["q"][:, :, ::2, :] = 0
+    prob["q"][:, :, ::2, 0] = 0x3F80               # 1
+    prob["q"][:, :, ::2, 1] = 0x3380               # 2^-24
+    prob["k"][..., 0] = 0x3F80 | rng.integers(0, 128, prob["k"].shape[:3])
+    prob["k"][..., 1] = 0x3F80
+    st = _check(prob, 0x3F800000)
+    n = int(prob["seq_len"].sum()) * rows          # half of the 2 rows query heads, each with every key
+    assert st["slow_path_scores"] >= n, (st, n)
+
+
+@pytest.mark.parametrize("rows", [4, 8, 16])
+def test_trees_and_bad_rows(gpu, rows):
+    """A tree mask across a step boundary; a NaN query row and an inf key flag exactly the rows that
+    see them, and a segment without keys is +0."""
+    rng = np.random.default_rng(50 + rows)
+    T, S, d = rows // 2, 100, 64
+    prob = _rand_problem(rng, "normal", "normal", B=3, T=T, Hq=4, Hkv=2, S=S, d=d, dv=d)
+    prob["seq_len"][:] = [S, 0, S]
+    prob["kv_len"][:] = np.repeat([70, 0, 0], T)
+    prob["tree_base"] = np.array([75, 0, 60], np.int32)
+    prob["tree_mask"] = rng.integers(0, 1 << 25, size=3 * T).astype(np.uint64) | np.uint64(1)
+    ab = default_alpha_bits(d)
+    _check(prob, ab)
+    prob["q"][0, T - 1, 1, 5] = 0x7FC0
+    prob["q"][1, 0, 0, 9] = 0xFF80   # a row without keys is still a domain error
+    prob["k"][2, 1, 60, 3] = 0x7F80  # tree key 0 of sequence 2, KV head 1: every row of heads 2, 3
+    clean = {k: (v.copy() if hasattr(v, "copy") else v) for k, v in prob.items()}
+    clean["q"][0, T - 1, 1, 5] = 0
+    clean["q"][1, 0, 0, 9] = 0
+    clean["k"][2, 1, 60, 3] = 0
+    want, _ = _oracle(clean, ab)
+    got, flags, st = _run(prob, ab)
+    exp = np.zeros((3, T, 4), np.uint8)
+    exp[0, T - 1, 1] = exp[1, 0, 0] = 2
+    exp[2, :, 2:] = 2
+    assert np.array_equal(flags.reshape(exp.shape), exp), (flags, st)
+    assert np.array_equal(got[exp == 0], want[exp == 0])
+
+
+def test_equal_share_plan(gpu):
+    """Ragged lengths on the equal-share plan, with shares that cross units, against the oracle and
+    one split; 200 sequences of few keys, so that most shares reach several units."""
+    ab = default_alpha_bits(128)
+    for B, S, Hq, T in ((200, 900, 8, 1), (16, 3000, 16, 2)):
+        rng = np.random.default_rng(B)
+        lens = rng.integers(T, S + 1, size=B)
+        lens[:2] = [S, T]
+        q, k, v = bf16(rng, (B, T, Hq, 128)), bf16(rng, (B, 2, S, 128), "outlier"), bf16(rng, (B, 2, S, 128))
+        prob = problem.contiguous(q, k, v, lens[:, None] - T + 1 + np.arange(T), seq_len=lens)
+        prob = problem.to_paged(prob, 16, rng)
+        want, _ = _oracle(prob, ab)
+        for splits in (0, 40, 1):
+            got, flags, st = _run(prob, ab, splits=splits)
+            assert st["decode_kernel_rows"] == flags.size and not flags.any(), st
+            assert splits != 40 or st["decode_equal_share_steps"] == 1, st
+            assert np.array_equal(got, want), st
