@@ -13,12 +13,13 @@
 // 25 per pair and lane for the certified weight.
 //
 // Measured against what ran before (MI355X, equal bits): 8 sequences of 16K keys, 16 rows, d = 128
-// 693 -> 226 us (ea_decode, 8 row blocks); 32 ragged sequences to 4K keys, 8 rows 228 -> 104 us;
+// 693 -> 220 us (ea_decode, 8 row blocks); 32 ragged sequences to 4K keys, 8 rows 228 -> 82 us;
 // 16 ragged sequences to 8K keys, 4 rows, d = 64 157 -> 41 us (ea_split); causal prefill of 2048
-// tokens, 32/8 heads, d = 64 2.89 -> 0.63 ms (ea_split).
+// tokens, 32/8 heads, d = 64 2.89 -> 0.61 ms (ea_split). The VALU's own time is 162 of the 220 us
+// (16 rows), 102 of 143 us (8 rows, 32 x 4K keys) and 65 of 115 us (4 rows, bound by memory).
 //
-// Waves per SIMD: a wave issues a VALU instruction at most every 8 cycles, the pipe takes one every
-// 4, so the variants whose registers allow it run 3 or 4 waves per SIMD (mr_waves).
+// The undecided pairs' exact path lives outside the step loop (a list in LDS, flush()): in it, its
+// registers spilled the loop's.
 //
 // Rounding: both instructions accumulate as a chain of four single-rounding FMAs in ascending k
 // order (checked bit for bit on the device against fma() chains), so the bounds are those of
@@ -61,6 +62,17 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// Waves per SIMD each variant is compiled for (512 registers per lane are shared among them), and
+// whether it keeps two steps of K and V in registers. A 4-row step is short, so its loads need the
+// longer lead: 32 x 4K keys, 4 rows 126 -> 115 us (4.7 TB/s) with two steps at 2 waves, 147 us at 4
+// waves, where the registers no longer hold one (scratch reads wait for every load before them). At
+// 8 and 16 rows one step is enough (143 and 220 us; 147 and 228 us with two). Non-temporal loads
+// cost 50% at 64 dims (a 128-byte line is read by two instructions) and nothing either way at 128.
+template <int RS, int DK>
+constexpr int mr_waves() { return RS == 16 && DK == 2 ? 3 : 2; }
+template <int RS>
+constexpr bool mr_two_steps() { return RS == 4; }
+
 template <int RS, int DK, int CPL>
 struct MRowSmem {
     static constexpr int QST = DK * 32 + 2;  // doubles per q row: 16 bytes of padding spread the rows over the banks
@@ -69,16 +81,14 @@ struct MRowSmem {
     double red[2][RS * 16 * CPL];
     double q1[RS];            // upper bound of sum |q_i|
     double wZ[4][RS];
-    int wR[4][RS], wn[4][RS];
+    int wR[4][RS], wf[4][RS];  // per wave: reference exponent, flag
+    int kvl[RS];               // rows' visible prefixes (rows past the segment: none) and tree masks
+    uint64_t tmk[RS];
     float vred[4][16];
     // pairs the score interval left undecided, per wave: (row, key). Flushed when MR_LIST are
     // waiting, so a step's 16 RS more always fit
-    int2 list[4][MR_LIST + 16 * RS];
+    int2 list[4][MR_LIST + (mr_two_steps<RS>() ? 32 : 16) * RS];
 };
-
-// waves per SIMD each variant is compiled for (512 registers per lane shared among them)
-template <int RS, int DK>
-constexpr int mr_waves() { return RS == 4 ? 4 : (RS == 8 ? 3 : (DK == 2 ? 3 : 2)); }
 
 // the larger of x and the values 16, 32 and 48 lanes away (lanes l, l ^ 16, l ^ 32, l ^ 48)
 __device__ __forceinline__ int max_x(int v) {
@@ -107,6 +117,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
     constexpr int NP = RS / 4;                 // pairs per lane and step
     constexpr int NR = RS == 16 ? 1 : NS;      // rows a lane holds in the score layout
     constexpr int NACC = RS / 4;               // row quads of the output layout
+    constexpr bool DB = mr_two_steps<RS>();
     typedef MRowSmem<RS, DK, CPL> Smem;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     Smem& S = *reinterpret_cast<Smem*>(smem_raw);
@@ -153,25 +164,22 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
             aq = wave_sum(aq);  // at most 128 terms in any order: times 1 + 2^-40 bounds the exact sum
             if (lane == 0) S.q1[r] = aq * (1.0 + 0x1p-40);
         }
-        // ---- the lane's rows in the score layout: row c (16 rows) or y + 4 s
+        // ---- the rows' visible keys: prefix and tree mask in LDS (steps inside every prefix do not
+        // read them), the last visible key and the shortest prefix of the block
         const int slen = P.seq_len[b];
         const int tb = P.tree_mask ? P.tree_base[b] : 0;
-        int kvl[NR];
-        uint64_t tmk[NR];
-        bool rvalid[NR];
         int kend = 0, kvmin = INT_MAX;
-#pragma unroll
-        for (int s = 0; s < NR; ++s) {
-            const int r = RS == 16 ? c : (c & 3) + 4 * s;
-            rvalid[s] = r < nrow;
-            const int lr = row0 + min(r, nrow - 1);
-            const int tok = b * P.g.num_tokens + lr / P.grp;
-            kvl[s] = P.kv_len[tok];
-            tmk[s] = P.tree_mask ? P.tree_mask[tok] : 0ull;
-            int e = kvl[s];
-            if (tmk[s]) e = max(e, tb + 64 - (int)__clzll(tmk[s]));
-            kend = max(kend, e);
-            kvmin = min(kvmin, kvl[s]);
+        {
+            const int r = lane & (RS - 1);
+            const int tok = b * P.g.num_tokens + (row0 + min(r, nrow - 1)) / P.grp;
+            const int kvl = P.kv_len[tok];
+            const uint64_t tmk = P.tree_mask ? P.tree_mask[tok] : 0ull;
+            kend = tmk ? max(kvl, tb + 64 - (int)__clzll(tmk)) : kvl;
+            kvmin = kvl;
+            if (w == 0 && lane < RS) {
+                S.kvl[r] = r < nrow ? kvl : INT_MIN;
+                S.tmk[r] = r < nrow ? tmk : 0ull;
+            }
         }
         kend = min(wave_max_dpp(kend), slen);
         kvmin = min(-wave_max_dpp(-kvmin), slen);
@@ -192,8 +200,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         const int voff = x * (int)vss2 + 2 * CPL * c;
         // 16 consecutive keys starting at a multiple of 16 lie in one page (page size >= 16)
         auto page_of = [&](int n) __attribute__((always_inline)) { return P.bt ? btb[min(n, k1 - 1) >> pshift] : b; };
-        u32x4 kr[DK], vr[4];
-        auto issue_k = [&](int n0, int pg) __attribute__((always_inline)) {
+        auto issue_k = [&](int n0, int pg, u32x4 (&kr)[DK]) __attribute__((always_inline)) {
             const int64_t sl = P.bt ? (n0 & pmask) : n0;
             const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
                 (void*)(kh + (int64_t)pg * kps2 + sl * kss2), (short)0, 0x7FFFFFFF, 0x00020000);
@@ -202,7 +209,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
             for (int j = 0; j < DK; ++j)
                 kr[j] = __builtin_amdgcn_raw_buffer_load_b128(rk, 8 * (4 * j + x) < kd ? koff + 64 * j : EA_OOB, 0, 0);
         };
-        auto issue_v = [&](int n0, int pg) __attribute__((always_inline)) {
+        auto issue_v = [&](int n0, int pg, u32x4 (&vr)[4]) __attribute__((always_inline)) {
             const int64_t sl = P.bt ? (n0 & pmask) : n0;
             const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
                 (void*)(vh + (int64_t)pg * vps2 + sl * vss2), (short)0, 0x7FFFFFFF, 0x00020000);
@@ -223,7 +230,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         // score bound per pair: |alpha| 66 u |q|_1 max|k| (the last factor per key), with slack for
         // the roundings of the products themselves
         double q1a[NR];
-        int R[NR], nv[NR];
+        int R[NR];
         double z[NR];
         int rfl = 0;  // bit s: the lane saw an undecided pair of its row s
         int n5 = 0, n6 = 0, n8 = 0, cnt = 0;  // wave-uniform
@@ -241,11 +248,15 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         for (int s = 0; s < NR; ++s) {
             q1a[s] = fabs(alpha) * (66.0 * 0x1p-53 * (1.0 + 0x1p-20)) * S.q1[RS == 16 ? c : (c & 3) + 4 * s];
             R[s] = MR_NONE;
-            nv[s] = 0;
             z[s] = 0.0;
         }
 
-        auto step = [&](int n0, int pgn) __attribute__((always_inline)) {
+        auto step = [&](int n0, int pgn, u32x4 (&kr)[DK], u32x4 (&vr)[4], u32x4 (&kn)[DK], u32x4 (&vn)[4]) __attribute__((always_inline)) {
+            if constexpr (DB) {
+                issue_k(n0 + 64, pgn, kn);
+                issue_v(n0 + 64, pgn, vn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // ---- scores
             double s_[NP];
             float km = 0.0f;
@@ -289,6 +300,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
                                 u1 = __builtin_amdgcn_mfma_f64_4x4x4f64(kf[2 * h + 1], qq[s][h].y, u1, 0, 0, 0);
                             }
                         }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (int p = 0; p < NP; ++p) {
@@ -298,9 +310,11 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
                 }
             }
             // K of the next step into the registers the scores are done with
-            __builtin_amdgcn_sched_barrier(0);
-            issue_k(n0 + 64, pgn);
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!DB) {
+                __builtin_amdgcn_sched_barrier(0);
+                issue_k(n0 + 64, pgn, kn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // ---- max |k| of the pairs' keys: over the 4 lanes of key c, then from the lane of the key
             const int kmx = max_x(__float_as_int(km));  // non-negative floats order as integers
             double adel[NP];
@@ -309,15 +323,15 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
             for (int p = 0; p < NP; ++p) {
                 const int key = (RS == 16 ? 4 * p : 4 * blk) + x;
                 adel[p] = q1a[RS == 16 ? 0 : p] * (double)__int_as_float(__shfl(kmx, key, 64));
-                vism |= rvalid[RS == 16 ? 0 : p] ? (1u << p) : 0u;
+                vism |= ((RS == 16 ? c : (c & 3) + 4 * p) < nrow) ? (1u << p) : 0u;
             }
             if (n0 + 16 > min(kvmin, k1)) {
                 vism = 0;
 #pragma unroll
                 for (int p = 0; p < NP; ++p) {
-                    const int s = RS == 16 ? 0 : p, n = n0 + (RS == 16 ? 4 * p : 4 * blk) + x, ti = n - tb;
-                    const bool in = ((unsigned)ti < 64u) & (((tmk[s] >> (ti & 63)) & 1ull) != 0);
-                    vism |= (rvalid[s] & (n < k1) & ((n < kvl[s]) | in)) ? (1u << p) : 0u;
+                    const int r = RS == 16 ? c : (c & 3) + 4 * p, n = n0 + (RS == 16 ? 4 * p : 4 * blk) + x, ti = n - tb;
+                    const bool in = ((unsigned)ti < 64u) & (((S.tmk[r] >> (ti & 63)) & 1ull) != 0);
+                    vism |= ((n < k1) & ((n < S.kvl[r]) | in)) ? (1u << p) : 0u;
                 }
             }
             // ---- certified weights
@@ -394,10 +408,10 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
                 if (g && far) rfl |= 1 << s;
                 om[p] = (g && !far) ? ldexp((double)M[p], de) : 0.0;
                 z[s] += om[p];
-                nv[s] += (vism >> p) & 1;
             }
             // ---- P.V
             auto pv = [&](auto ic) __attribute__((always_inline)) {
+                __builtin_amdgcn_sched_barrier(0);
                 constexpr int i = decltype(ic)::value;
                 double wr[NS];
                 if constexpr (RS != 16) {
@@ -425,9 +439,11 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
             pv(std::integral_constant<int, 1>{});
             pv(std::integral_constant<int, 2>{});
             pv(std::integral_constant<int, 3>{});
-            __builtin_amdgcn_sched_barrier(0);
-            issue_v(n0 + 64, pgn);
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!DB) {
+                __builtin_amdgcn_sched_barrier(0);
+                issue_v(n0 + 64, pgn, vn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         };
 
         // ---- the pairs waiting in the list: every product of the score separately, TwoSum-accumulated
@@ -547,24 +563,29 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         };
 
         // ---- the wave's steps: K of the next one is requested once the scores have read this one's
-        // registers, V once P.V has; pages are looked up a step ahead
-        if (nst > 0) {
-            int pg = page_of(k0w);
-            issue_k(k0w, pg);
-            issue_v(k0w, pg);
-            pg = page_of(k0w + 64);
-            int it = 0;
+        // registers, V once P.V has; pages are looked up a step ahead. A flush (rare) drops the
+        // loads in flight, so that their registers are not live across it, and starts over
+        for (int it = 0; it < nst;) {
+            u32x4 ka[DK], va[4], kb[DK], vb[4];
+            int pg = page_of(k0w + 64 * it);
+            issue_k(k0w + 64 * it, pg, ka);
+            issue_v(k0w + 64 * it, pg, va);
+            pg = page_of(k0w + 64 * it + 64);
 #pragma unroll 1
-            do {
-#pragma unroll 1
-                for (; it < nst && cnt < MR_LIST; ++it) {
-                    const int n0 = k0w + 64 * it;
-                    const int pgn = pg;
-                    pg = page_of(n0 + 128);
-                    step(n0, pgn);
+            for (; it < nst && cnt < MR_LIST; it += DB ? 2 : 1) {
+                const int n0 = k0w + 64 * it;
+                int pgn = pg;
+                pg = page_of(n0 + 128);
+                if constexpr (DB) {
+                    step(n0, pgn, ka, va, kb, vb);
+                    pgn = pg;
+                    pg = page_of(n0 + 192);
+                    if (it + 1 < nst) step(n0 + 64, pgn, kb, vb, ka, va);
+                } else {
+                    step(n0, pgn, ka, va, ka, va);
                 }
-                if (cnt > 0) flush();
-            } while (it < nst);
+            }
+            if (cnt > 0) flush();
         }
 
         // ---- epilogue: row totals of the wave, then the 4 waves' partials at the rows' largest
@@ -572,26 +593,22 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
 #pragma unroll
         for (int s = 0; s < NR; ++s) {
             double zs = z[s];
-            int ns = nv[s], fl = (rfl >> s) & 1;
+            int fl = (rfl >> s) & 1;
             if constexpr (RS != 16) {
                 zs += __shfl_xor(zs, 4, 64);
-                ns += __shfl_xor(ns, 4, 64);
                 fl |= __shfl_xor(fl, 4, 64);
                 zs += __shfl_xor(zs, 8, 64);
-                ns += __shfl_xor(ns, 8, 64);
                 fl |= __shfl_xor(fl, 8, 64);
             }
             zs += __shfl_xor(zs, 16, 64);
-            ns += __shfl_xor(ns, 16, 64);
             fl |= __shfl_xor(fl, 16, 64);
             zs += __shfl_xor(zs, 32, 64);
-            ns += __shfl_xor(ns, 32, 64);
             fl |= __shfl_xor(fl, 32, 64);
             if (RS == 16 ? x == 0 : (x == 0 && blk == 0)) {
                 const int r = RS == 16 ? c : c + 4 * s;
                 S.wR[w][r] = R[s];
                 S.wZ[w][r] = zs;
-                S.wn[w][r] = fl ? -1 : ns;
+                S.wf[w][r] = fl;
             }
         }
         vmx = __int_as_float(max_x(__float_as_int(vmx)));
@@ -611,7 +628,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
                 if constexpr (RS == 16) acc[i][e] = acc16[e][i] * f;
                 else acc[i][e] *= f;
             }
-            if (far4 >> i & 1 && c == 0) S.wn[w][r] = -1;
+            if (far4 >> i & 1 && c == 0) S.wf[w][r] = 1;
         }
         auto put = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -647,13 +664,15 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         } else if (w == 1) {
             if (lane < nrow) {
                 const int r = lane;
-                int Rm = MR_NONE, n = 0;
-                bool fl = false;
+                int Rm = MR_NONE, fl = 0;
                 for (int ww = 0; ww < 4; ++ww) {
                     Rm = max(Rm, S.wR[ww][r]);
-                    fl |= S.wn[ww][r] < 0;
-                    n += S.wn[ww][r];
+                    fl |= S.wf[ww][r];
                 }
+                // keys of the piece up to the row's last visible one: at least the keys summed
+                const uint64_t tm = S.tmk[r];
+                const int ke = min(tm ? max(S.kvl[r], tb + 64 - (int)__clzll(tm)) : S.kvl[r], k1);
+                const int n = Rm == MR_NONE ? 0 : ke - kA;
                 double zs[4];
                 for (int ww = 0; ww < 4; ++ww)
                     zs[ww] = S.wR[ww][r] == MR_NONE ? 0.0 : ldexp(S.wZ[ww][r], max(S.wR[ww][r] - Rm, -1000));
