@@ -365,7 +365,8 @@ __device__ __forceinline__ void decode_body(Params P) {
                 if ((lane & 15) == 0) S.qnb[r][lane >> 4] = qb;
             }
             // the step's first kernel on this path clears the tier-2 work list and chunk counts
-            if (item == 0 && split == 0 && lane <= EA_T2_BLOCKS) P.wl_cnt[lane] = 0;
+            if (item == 0 && split == 0)
+                for (int i = lane; i < EA_T2_CNT; i += 64) P.wl_cnt[i] = 0;
             wait_vm<0>();  // the q stores are complete before the barrier
         }
         __syncthreads();  // tables visible

@@ -27,6 +27,7 @@
 #include "ea_params.h"
 #include "ea_combine.h"
 #include "ea_exact.h"
+#include "ea_refine.h"
 
 using namespace ea;
 
@@ -94,12 +95,12 @@ __device__ void dq_plan_block(const Params& P) {
 
 // The equal-share plan alone (the multi-row kernel's steps), and the cleared tier-2 work list.
 __global__ void __launch_bounds__(1024) ea_plan(Params P) {
-    if (threadIdx.x <= EA_T2_BLOCKS) P.wl_cnt[threadIdx.x] = 0;
+    if (threadIdx.x < EA_T2_CNT) P.wl_cnt[threadIdx.x] = 0;
     dq_plan_block<1024>(P);
 }
 
 __global__ void __launch_bounds__(256) ea_prep(Params P) {
-    if (blockIdx.x == 0 && threadIdx.x <= EA_T2_BLOCKS) P.wl_cnt[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < EA_T2_CNT) P.wl_cnt[threadIdx.x] = 0;
     if (P.dq_stream && blockIdx.x == gridDim.x - 1) {
         dq_plan_block<256>(P);  // the extra last block
         return;
@@ -670,21 +671,19 @@ struct T2Part {
     uint64_t nhi[EA_MAXDV], nlo[EA_MAXDV], ner[EA_MAXDV];  // N_c,b in units 2^(nr_c - F), lost count
 };
 
-// Rows are split into C key chunks when fewer rows are listed than there are blocks (C = blocks /
-// rows, so one flagged row takes every block instead of one): block (row slot, chunk) computes the
+// The listed rows in 128-bit arithmetic, by blocks bid, bid + nb, ... Rows are split into C key
+// chunks when fewer rows are listed than there are blocks (C = blocks / rows, so one flagged row
+// takes every block instead of one): block (row slot, chunk) computes the
 // chunk's logits and weights and its Z and N sums, writes them as a T2Part, and the row's last
 // chunk block to finish merges the C partials. Merging moves each floored partial to the row's
 // larger base by an arithmetic right shift: floor(a 2^-s) <= a 2^-s < floor(a 2^-s) + lost, so
 // the row's sums stay of the form [acc, acc + lost count] in units of the common base, the form
-// the final rounding takes. With C = 1 the block finishes the row itself.
-__global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
-    __shared__ T2Smem S;
-    __shared__ int s_last;
+// the final rounding takes. With C = 1 the block finishes the row itself. left: only the rows that
+// the double-double pass marked (C = 1).
+__device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last, int cnt, int C, int bid, int nb, bool left) {
     const int tid = threadIdx.x;
-    const int cnt = *P.wl_cnt;
-    const int C = cnt >= (int)gridDim.x ? 1 : (int)gridDim.x / max(cnt, 1);
     const int64_t items = (int64_t)cnt * C;
-    if ((int64_t)blockIdx.x >= items) return;  // no listed row for this block (the usual case)
+    if ((int64_t)bid >= items) return;
     for (int i = tid; i < 256; i += EA_T2_THREADS) {
         S.T1[i] = u64_as_f64(EA_T1_BITS[i]);
         S.T2[i] = u64_as_f64(EA_T2_BITS[i]);
@@ -692,12 +691,14 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
     __syncthreads();
     const int d = P.g.head_dim, dv = P.g.head_dim_v;
     const int Hq = P.g.num_q_heads, T = P.g.num_tokens;
-    int32_t* Mw = P.t2M + (int64_t)blockIdx.x * P.t2_keys;
-    int64_t* Ew = P.t2E + (int64_t)blockIdx.x * P.t2_keys;
+    int32_t* Mw = P.t2M + (int64_t)bid * P.t2_keys;
+    int64_t* Ew = P.t2E + (int64_t)bid * P.t2_keys;
     T2Part* parts = (T2Part*)P.t2part;
-    for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+    for (int64_t item = bid; item < items; item += nb) {
         const int slot = (int)(item / C), chunk = (int)(item % C);
-        const int64_t row = P.wl[slot];
+        const int32_t entry = agent_load(&P.wl[slot]);
+        const int64_t row = entry & 0x7FFFFFFF;
+        if (left && entry >= 0) continue;
         const int64_t b = row / ((int64_t)T * Hq);
         const int t = (int)((row / Hq) % T), hq = (int)(row % Hq);
         const int hk = hq / P.grp;
@@ -1092,6 +1093,42 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
     }
 }
 
+// Tier 2: the listed rows in double-double (ea_refine.h), in EA_DD_PARTS key chunks in all when few
+// rows are listed; then, where a row stays undecided, the last block to finish takes what is left in
+// 128-bit arithmetic. force_tier2 sends every row straight to the 128-bit path, over EA_T2_BLOCKS
+// blocks. Measured: the 70 rows that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
+// 4096-key bf16 row after a prefill step 116 -> 35 us; an empty list 4.0-4.5 us
+// in the trace; 512 blocks cost a C2 step 1.8 us, so bf16 steps, which list few rows, launch 32.
+__global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
+    __shared__ union {
+        T2Smem t2;
+        DDSmem dd;
+    } S;
+    __shared__ int s_last;
+    const int cnt = *P.wl_cnt;
+    if (cnt == 0) return;  // the usual case
+    if (P.t2_force) {
+        t2_rows(P, S.t2, s_last, cnt, cnt >= EA_T2_BLOCKS ? 1 : EA_T2_BLOCKS / cnt, (int)blockIdx.x, EA_T2_BLOCKS, false);
+        return;
+    }
+    // every item of a split row is in flight at once (a block each, a partial each, a count per row)
+    // and no chunk is shorter than a pass of 128 keys
+    const int C = cnt <= EA_T2_ROWS ? min(min(EA_DD_PARTS, (int)gridDim.x) / cnt, (P.t2_keys + EA_DD_KEYS - 1) / EA_DD_KEYS) : 1;
+    dd_rows(P, S.dd, cnt, max(C, 1), (DDPart*)P.ddpart);
+    // the last of the blocks that had a row takes the rows left over: their marks in the list and their
+    // count are atomics, complete before the block's own count
+    const int64_t items = (int64_t)cnt * max(C, 1);
+    if ((int64_t)blockIdx.x >= items) return;
+    agent_done();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = atomicAdd(&P.wl_cnt[EA_T2_DONE], 1) == (int)min(items, (int64_t)gridDim.x) - 1 &&
+                 agent_load(&P.wl_cnt[EA_T2_LEFT]) != 0;
+    __syncthreads();
+    if (!s_last) return;
+    t2_rows(P, S.t2, s_last, cnt, 1, 0, 1, true);
+}
+
 // Lists every row for tier 2 (ea_options.force_tier2); runs after tier 1, so nothing else appends.
 __global__ void __launch_bounds__(256) ea_list_all(Params P) {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1387,14 +1424,16 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     pl->off_pN = off; off = align_up(off + (size_t)pl->nsplit * R * dv * 8);
     pl->off_pV = off; off = align_up(off + (size_t)pl->nsplit * pl->nseg * std::max(pl->nrb, pl->gen_nrb) * dv * 4);
     pl->off_wl = off; off = align_up(off + (size_t)(R > 0 ? R : 1) * 4);
-    pl->off_cnt = off; off = align_up(off + 4 * (1 + EA_T2_BLOCKS));
+    pl->off_cnt = off; off = align_up(off + 4 * EA_T2_CNT);
     pl->off_t2part = off; off = align_up(off + EA_T2_BLOCKS * sizeof(T2Part));
     pl->off_dq = off;
     pl->dq_rec_off = (3 + pl->dq_units + 3) & ~3;  // 16-byte aligned block records after S
     if (pl->dq) off = align_up(off + (size_t)(pl->dq_rec_off + 4 * EA_DQ_MAX_BLOCKS) * 4);
     pl->t2_keys = maxlen + 64;
     pl->off_t2M = off; off = align_up(off + (size_t)EA_T2_BLOCKS * pl->t2_keys * 4);
-    pl->off_t2E = off; off = align_up(off + (size_t)EA_T2_BLOCKS * pl->t2_keys * 8);
+    // the double-double chunk partials share the 128-bit path's key scratch (never in use together)
+    pl->off_t2E = off;
+    off = align_up(off + std::max((size_t)EA_T2_BLOCKS * pl->t2_keys * 8, EA_DD_PARTS * sizeof(DDPart)));
     pl->prefill = ea_prefill_eligible(*g, pl->grp, o->kernel, &pl->pf_ntiles, &pl->pf_nrb) ? 1 : 0;
     pl->off_pfq = pl->off_pfqm = pl->off_pfkv = pl->off_pfscr = pl->off_pfpart = 0;
     pl->pf_nsplit = pl->pf_tps = 1;
@@ -1544,6 +1583,8 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     P.t2part = (void*)(ws + pl.off_t2part);
     P.t2M = (int32_t*)(ws + pl.off_t2M);
     P.t2E = (int64_t*)(ws + pl.off_t2E);
+    P.ddpart = (void*)(ws + pl.off_t2E);
+    P.t2_force = o->force_tier2 ? 1 : 0;
     P.t2_keys = pl.t2_keys;
     P.pfq = (uint8_t*)(ws + pl.off_pfq);
     P.pfqm = (void*)(ws + pl.off_pfqm);
@@ -1619,7 +1660,7 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         if ((rc = mark(3))) return rc;
         if (o->tier2) {
             if ((rc = list_all(P, o, rb4 * 4 / 256 + 1, st))) return rc;
-            hipLaunchKernelGGL(ea_tier2, dim3(EA_T2_BLOCKS), dim3(EA_T2_THREADS), 0, st, P);
+            hipLaunchKernelGGL(ea_tier2, dim3(P.t2_force ? EA_T2_BLOCKS : EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
             rc = herr(hipGetLastError());
             if (rc) return rc;
         }
@@ -1681,7 +1722,7 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     if ((rc = mark(3))) return rc;
     if (o->tier2) {
         if ((rc = list_all(P, o, rb4 * 4 / 256 + 1, st))) return rc;
-        hipLaunchKernelGGL(ea_tier2, dim3(EA_T2_BLOCKS), dim3(EA_T2_THREADS), 0, st, P);
+        hipLaunchKernelGGL(ea_tier2, dim3(P.t2_force ? EA_T2_BLOCKS : EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
         rc = herr(hipGetLastError());
         if (rc) return rc;
     }

@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
     S.T2[tid] = u64_as_f64(EA_T2_BITS[tid]);
     if (blockIdx.x == 0 && blockIdx.y == 0) {
         // on uniform splits the step's first kernel clears the tier-2 work list and chunk counts
-        if (!P.dq_stream && tid <= EA_T2_BLOCKS) P.wl_cnt[tid] = 0;
+        if (!P.dq_stream && tid < EA_T2_CNT) P.wl_cnt[tid] = 0;
         if (tid == 0 && P.stats) atomicAdd((unsigned long long*)&P.stats[9], (unsigned long long)P.rows);
     }
 

@@ -13,7 +13,14 @@ namespace ea {
 #define EA_MAXRB 4
 #define EA_MAXD 128
 #define EA_MAXDV 128
-#define EA_T2_BLOCKS 32
+#define EA_T2_BLOCKS 32             // blocks of tier 2's 128-bit path
+// tier 2's counters (Params::wl_cnt): rows listed, chunks done per row (of the first EA_T2_ROWS), rows
+// the double-double pass left undecided, blocks that finished it
+#define EA_T2_ROWS 192
+#define EA_T2_LEFT (1 + EA_T2_ROWS)
+#define EA_T2_DONE (2 + EA_T2_ROWS)
+#define EA_T2_CNT (3 + EA_T2_ROWS)
+#define EA_DD_BLOCKS(fp32) ((fp32) ? 512 : 32)  // of the double-double pass: two per CU where many rows are listed
 
 // ------------------------------------------------------------------------------------------------
 // Kernel parameters
@@ -52,11 +59,13 @@ struct Params {
     double* pN;       // nsplit * rows * dv
     float* pV;        // nsplit * nseg * nrb * dv : max |v| per channel over the block's keys
     int32_t* wl;      // rows
-    int32_t* wl_cnt;  // 1 + EA_T2_BLOCKS: the work list's length, then tier 2's per-row chunk counts
+    int32_t* wl_cnt;  // EA_T2_CNT counters of tier 2
     void* t2part;     // EA_T2_BLOCKS tier-2 chunk partials (T2Part, ea_hip.hip)
     int32_t* t2M;     // EA_T2_BLOCKS * max_keys
     int64_t* t2E;     // EA_T2_BLOCKS * max_keys
+    void* ddpart;     // EA_DD_PARTS chunk partials of the double-double pass (DDPart, ea_refine.h)
     int32_t t2_keys;
+    int32_t t2_force;  // 1: every row is listed, straight for the 128-bit path
     // int8-MFMA prefill path (ea_prefill.hip)
     uint8_t* pfq;     // rows * 512: q digit planes
     void* pfqm;       // rows * sizeof(PfQMeta)

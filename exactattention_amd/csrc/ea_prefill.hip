@@ -240,7 +240,7 @@ __device__ __forceinline__ void slice32(const uint16_t* src, bool valid, Slice32
 // work-list counter (this is the step's first kernel on the prefill path).
 // ------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) ea_pf_qslice(Params P) {
-    if (blockIdx.x == 0 && threadIdx.x <= EA_T2_BLOCKS) P.wl_cnt[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < EA_T2_CNT) P.wl_cnt[threadIdx.x] = 0;
     const int q16 = threadIdx.x & 15;
     const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
     if (row >= P.rows) return;  // whole 16-lane groups leave together

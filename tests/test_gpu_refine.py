@@ -1,0 +1,88 @@
+"""Tier 2's double-double pass (ea_refine.h): rows that tier 1 lists are certified there, or go on to
+the 128-bit path; either way the bits are the oracle's."""
+
+import numpy as np
+import pytest
+
+from exactattention_amd.formats import default_alpha_bits
+from test_gpu_parity import _oracle, _rand_problem, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,S,kind", [(300, 300, "normal"), (70, 1000, "normal"), (64, 130, "outlier"), (96, 200, "dupes"),
+                                      (80, 129, "wide")])
+def test_many_listed_rows(gpu, T, S, kind):
+    """fp32 outputs of the int8 prefill kernel with logits 4 times the usual scale: its bounds leave
+    many rows, more than the pass has chunk counters for, so blocks take whole rows. dupes: sums
+    that are exact and quotients that tie."""
+    rng = np.random.default_rng(T + S)
+    prob = _rand_problem(rng, kind, kind, B=1, T=T, Hq=2, Hkv=1, S=S, d=128, dv=128)
+    ab = int(np.float32(0.5).view(np.uint32))
+    want, wflags = _oracle(prob, ab, "fp32")
+    got, flags, st = _run(prob, ab, "fp32")
+    assert not np.any(wflags) and not flags.any(), st
+    assert np.array_equal(got, want), st
+    assert st["tier2_certified"] == st["tier1_flagged"], st
+    if kind == "normal":
+        assert st["tier1_flagged"] > 32, st
+
+
+@pytest.mark.parametrize("d,dv", [(128, 128), (64, 64), (40, 6)])
+@pytest.mark.parametrize("S", [1, 127, 129, 5000])
+def test_few_listed_rows(gpu, d, dv, S):
+    """Rows that cancel to about 2^-45 of their terms in some channels fail tier 1's bound whatever
+    the kernel: few of them, so their keys are split into chunks; a chunk without keys, tree keys,
+    misaligned rows. Their neighbours are certified by tier 1."""
+    rng = np.random.default_rng(d + S)
+    prob = _rand_problem(rng, "normal", "normal", B=2, T=1, Hq=2, Hkv=2, S=S + 60, d=d, dv=dv)
+    prob["seq_len"][:] = S + 60
+    prob["kv_len"][:] = S
+    prob["tree_base"] = np.full(2, S, np.int32)
+    prob["tree_mask"] = np.array([(1 << 59) | 5, 0], np.uint64)
+    # sequence 0, head 0: q = 0, so all weights are equal; channel 0 sums to one small element
+    prob["q"][0, 0, 0] = 0
+    n = S + 3  # its visible keys
+    col = np.zeros(n, np.uint16)
+    col[0:n - 1:2], col[1:n:2] = 0x3FC0, 0xBFC0  # 1.5, -1.5, ...
+    if n % 2:
+        col[n - 1] = 0
+    col[n // 2] = (0x2C00 if col[n // 2] == 0 else col[n // 2])
+    keys = np.concatenate([np.arange(S), S + np.array([0, 2, 59])])
+    prob["v"][0, 0, keys, 0] = col
+    if n > 2:
+        prob["v"][0, 0, keys[n - 1], 0] = 0x2C00  # about 2^-39
+        if n % 2 == 0:
+            prob["v"][0, 0, keys[n - 2], 0] = 0
+    ab = default_alpha_bits(d)
+    for out in ("bf16", "fp32"):
+        want, wflags = _oracle(prob, ab, out)
+        got, flags, st = _run(prob, ab, out)
+        assert not np.any(wflags) and not flags.any(), st
+        assert np.array_equal(got, want), st
+        assert st["tier2_certified"] == st["tier1_flagged"], st
+
+
+def test_domain_errors_among_listed_rows(gpu):
+    """NaN/inf in q, K and V, an fp32 logit overflow and a row without keys, beside rows the pass
+    certifies: exactly those that see a bad value are flag 2, +0."""
+    rng = np.random.default_rng(9)
+    T = 70
+    prob = _rand_problem(rng, "normal", "normal", B=1, T=T, Hq=2, Hkv=1, S=400, d=128, dv=128)
+    prob["seq_len"][:] = 400
+    prob["kv_len"][:] = 200 + np.arange(T)
+    prob["kv_len"][3] = 0
+    ab = int(np.float32(0.5).view(np.uint32))
+    want, _ = _oracle(prob, ab, "fp32")
+    prob["q"][0, 3, 0, 1] = 0x7FC0   # without keys: still a domain error
+    prob["q"][0, 10, 1, 0] = 0xFF80
+    prob["k"][0, 0, 250, 5] = 0x7FC0  # tokens 51 ..
+    prob["v"][0, 0, 260, 7] = 0x7F80  # tokens 61 ..
+    prob["q"][0, 20, 0, :] = 0x7F00   # about 2^127 per element: the logit overflows
+    got, flags, st = _run(prob, ab, "fp32")
+    exp = np.zeros((T, 2), np.uint8)
+    exp[3, 0] = exp[10, 1] = exp[20, 0] = 2
+    exp[51:] = 2
+    assert np.array_equal(flags.reshape(T, 2), exp), st
+    ok = exp[None] == 0
+    assert np.array_equal(got[ok], want[ok]) and not got[~ok].any(), st
