@@ -1,5 +1,5 @@
-// Merge of the KV-split partials of one row and the certified final rounding (one wave per row;
-// the combine kernel in ea_hip.hip).
+// Merge of the KV-split partials of one row and the certified final rounding (one wave per row; the
+// combine kernel in ea_hip.hip).
 #pragma once
 #include "ea_params.h"
 
@@ -8,7 +8,9 @@ namespace ea {
 // Returns the row's stats events, the same in every lane: bit 0 the row was merged (stats[0]),
 // bit 1 it is flagged (stats[1]), bit 2 only its final rounding failed (stats[7]). The caller
 // adds them up per block.
+template <int PRE>
 __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
+    constexpr int SLAB = 2 * PRE;  // splits per load round past PRE of them
     const int dv = P.g.head_dim_v;
     const int Hq = P.g.num_q_heads, T = P.g.num_tokens;
     const int64_t b = row / ((int64_t)T * Hq);
@@ -43,17 +45,17 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
         mo_ok = seen == (ns == 64 ? ~0ull : ((1ull << ns) - 1));
         if (mo_ok) si = m;
     }
-    // up to 8 splits in index order: every channel partial of both lane channels is requested
+    // up to PRE splits in index order: every channel partial of both lane channels is requested
     // now, in the same round as the split scalars (one load latency per row instead of three);
     // splits that turn out empty are dropped by selects below
-    const bool pre = ns <= 8 && !mo_ok && dv <= 128;
-    double pfn[2][8];
-    float pfv[2][8];
+    const bool pre = ns <= PRE && !mo_ok && dv <= 128;
+    double pfn[2][PRE];
+    float pfv[2][PRE];
     if (pre) {
 #pragma unroll
         for (int ci = 0; ci < 2; ++ci)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
+            for (int k = 0; k < PRE; ++k) {
                 const int c = lane + 64 * ci;
                 const bool in = k < ns && c < dv;
                 const int64_t o = (int64_t)k * P.rows + row;
@@ -74,6 +76,7 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
             *z = P.pZ[o];
         }
     };
+    const int qflag = P.mrow ? 0 : P.qinfo[row * 5 + 4];  // requested with the scalars below
     int n0, r0;
     double z0;
     load_split(0, &n0, &r0, &z0);
@@ -88,10 +91,8 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
     const int R = wave_max_i(R_l);
     // a NaN/inf in q flags the row. Partials with keys carry that flag already when the multi-row
     // kernel wrote them (no score of such a row is finite); a row without keys is looked at here
-    bool qbad = false;
-    if (!P.mrow) {
-        qbad = P.qinfo[row * 5 + 4] != 0;
-    } else if (R == INT_MIN) {
+    bool qbad = qflag != 0;
+    if (P.mrow && R == INT_MIN) {
         const uint16_t* qr = P.q + b * P.g.q_seq_stride + (int64_t)t * P.g.q_tok_stride + (int64_t)hq * P.g.q_head_stride;
         bool nf = false;
         for (int i = lane; i < P.g.head_dim; i += 64) nf |= ((qr[i] >> 7) & 0xFF) == 0xFF;
@@ -157,9 +158,9 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
     };
     const int dsh0 = shift_of(n0, r0);
     if (pre) {
-        int nk[8], shk[8];
+        int nk[PRE], shk[PRE];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < PRE; ++k) {
             nk[k] = __shfl(n0, k, 64);
             shk[k] = __shfl(dsh0, k, 64);
         }
@@ -172,7 +173,7 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
                 double N = 0.0;
                 float vmaxf = 0.0f;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
+                for (int k = 0; k < PRE; ++k) {
                     const bool use = k < ns && nk[k] > 0;
                     N += use ? ldexp(pfn[ci][k], max(shk[k], -1000)) : 0.0;
                     const float vm = use ? pfv[ci][k] : 0.0f;
@@ -185,7 +186,7 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
             else o16[obase + c] = (uint16_t)bits;
         }
     } else {
-        // per slab, both lane channels of 16 splits requested per round: a row of 32 splits waits
+        // per slab, both lane channels of SLAB = 16 splits requested per round: a row of 32 splits waits
         // for 2 load latencies, of 64 for 4, and each further slab adds one for its scalars
         double N[2] = {0.0, 0.0};
         float vmaxf[2] = {0.0f, 0.0f};
@@ -200,12 +201,12 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
                     dj = shift_of(nj, r);
                 }
                 const int cnt = min(64, ns - 64 * j);
-                for (int i0 = 0; i0 < cnt; i0 += 16) {
-                    double pn[2][16];
-                    float pv[2][16];
-                    int sh[16];
+                for (int i0 = 0; i0 < cnt; i0 += SLAB) {
+                    double pn[2][SLAB];
+                    float pv[2][SLAB];
+                    int sh[SLAB];
 #pragma unroll
-                    for (int k = 0; k < 16; ++k) {
+                    for (int k = 0; k < SLAB; ++k) {
                         const int i = i0 + k;
                         const int s = __shfl(sj, i & 63, 64), n = __shfl(nj, i & 63, 64);
                         sh[k] = __shfl(dj, i & 63, 64);
@@ -220,7 +221,7 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
                         }
                     }
 #pragma unroll
-                    for (int k = 0; k < 16; ++k)
+                    for (int k = 0; k < SLAB; ++k)
 #pragma unroll
                         for (int ci = 0; ci < 2; ++ci) {
                             N[ci] += ldexp(pn[ci][k], max(sh[k], -1000));

@@ -578,13 +578,17 @@ __global__ void __launch_bounds__(EA_THREADS, 2) ea_split(Params P) {
 // (D_s + nsplit):
 //   eZ = u' A + tiny,  eN_c = u' A max_s Vmax_sc + tiny.
 // ------------------------------------------------------------------------------------------------
+// PRE: the splits whose partials are requested in one round with their scalars. A decode step has few
+// rows of many splits, and 8 in a round; a step of many rows (prefill) has one or two pieces per
+// row and wants waves in flight instead (PRE 2: 72 registers against 157; 65,536 rows 95 -> 55 us).
+template <int PRE>
 __global__ void __launch_bounds__(64) ea_combine(Params P) {
     // one row per 64-thread block: the merge is a chain of dependent loads, so it wants as many
     // rows in flight as the machine holds. stats[0] counts the step's rows once; the per-row
     // counters only move for flagged rows (rare), so they never serialise on one address.
     const int64_t row = blockIdx.x;
     if (row == 0 && threadIdx.x == 0 && P.stats) atomicAdd((unsigned long long*)&P.stats[0], (unsigned long long)P.rows);
-    const int ev = combine_row(P, row, threadIdx.x);
+    const int ev = combine_row<PRE>(P, row, threadIdx.x);
     if (threadIdx.x == 0 && P.stats && (ev & 2)) {
         atomicAdd((unsigned long long*)&P.stats[1], 1ull);
         if (ev & 4) atomicAdd((unsigned long long*)&P.stats[7], 1ull);
@@ -1297,14 +1301,21 @@ struct Plan {
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Rows per block of the multi-row kernel for this geometry, 0 where another kernel takes the step.
-// d = dv = 128: from 3 rows per segment on (1 and 2 rows are what ea_decode's 2-row blocks are for:
-// 32 x 4K keys 108 us there) up to where the int8 prefill kernel starts. Any other head size: always
-// (ea_split takes what the pointers or pages do not allow).
+// d = dv = 128: from 3 rows per segment on, up to where the int8 prefill kernel starts. With 1 or 2
+// rows ea_decode (whose 2-row blocks read at the rate of a large copy) takes the steps of 4096 or more
+// segment tiles, and this kernel, with half its tile latency (1.9 against 3.5 us) and splits down to
+// a tile, the shorter ones. 16/8 heads, the step's kernels, ea_decode -> here: 1 x 300 keys 36.6 ->
+// 17.2 us, 1 x 4K 39.8 -> 28, 16 x 1K 44.9 -> 40.4, 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134,
+// 32 x 4K 117 -> 131. Any other head size: always (ea_split takes what the pointers or pages do not
+// allow).
 int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {
     if (o->timers || o->kernel == EA_KERNEL_GENERAL) return 0;
     if (g->head_dim == 128 && g->head_dim_v == 128) {
         int nt = 0, nr = 0;
-        if (r_seg <= 2 || ea_prefill_eligible(*g, g->num_q_heads / g->num_kv_heads, o->kernel, &nt, &nr)) return 0;
+        const int64_t tiles = (int64_t)g->num_seqs * g->num_kv_heads * (((int64_t)g->max_seq_len + 63) / 64);
+        if ((r_seg <= 2 && tiles >= 4096) ||
+            ea_prefill_eligible(*g, g->num_q_heads / g->num_kv_heads, o->kernel, &nt, &nr))
+            return 0;
     }
     return r_seg <= 4 ? 4 : (r_seg <= 8 ? 8 : 16);
 }
@@ -1336,7 +1347,8 @@ void choose_splits(int64_t items, int maxlen, int splits, int* nsplit, int* spli
 }
 
 // The same for the multi-row kernel. First enough blocks to fill the device, down to one tile per
-// split: a short context then takes a step or two per wave instead of a chain of them. Then splits
+// split (two from 16 splits on: merging 64 splits costs 16 us, 32 splits 10): a short context then
+// takes a step or two per wave instead of a chain of them. Then splits
 // of at most 512 keys, so that the equal-share plan (taken past one round of resident blocks) can
 // even out sequences of different lengths in shares of 8 tiles, while the partials stay below
 // MROW_PART and the workspace below the allocation-free entry point's array.
@@ -1348,7 +1360,7 @@ void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsp
         const int64_t items = pl.r_seg <= 8 ? (int64_t)pl.nseg * ((pl.r_seg + 1) / 2) : 2 * units;
         const int64_t rest = (int64_t)EA_T2_BLOCKS * 12 * maxlen + pl.rows * 1100;
         ns = 1;
-        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 64) ns *= 2;
+        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= (ns >= 8 ? 128 : 64)) ns *= 2;
         while ((int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART &&
                2 * ns * pl.rows * dv * 8 + rest <= MROW_WS)
             ns *= 2;
@@ -1407,7 +1419,7 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     pl->dq = (pl->mrow || (g->head_dim == 128 && g->head_dim_v == 128)) && o->kernel != EA_KERNEL_GENERAL &&
              !o->timers && !ea_prefill_eligible(*g, pl->grp, o->kernel, &pf_nt, &pf_nr) && pl->rows < ((int64_t)1 << 30) &&
              (int64_t)maxlen + 64 < ((int64_t)1 << 30) &&
-             (int64_t)pl->nseg * max_nrb * max_tiles < ((int64_t)1 << 30) &&
+             (int64_t)pl->nseg * max_nrb * std::max<int64_t>(max_tiles, 1) < ((int64_t)1 << 30) &&
              (int64_t)pl->nseg * max_nrb < ((int64_t)1 << 24);
     pl->dq_units = (int)std::min<int64_t>(pl->nseg * max_nrb, 1 << 24);
     pl->dq_max_tiles = (int)max_tiles;
@@ -1716,7 +1728,8 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         return rc;
     }
     if ((rc = mark(2))) return rc;
-    hipLaunchKernelGGL(ea_combine, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
+    if (pl.rows >= 8192) hipLaunchKernelGGL(ea_combine<2>, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
+    else hipLaunchKernelGGL(ea_combine<8>, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
     rc = herr(hipGetLastError());
     if (rc) return rc;
     if ((rc = mark(3))) return rc;

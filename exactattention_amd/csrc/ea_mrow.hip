@@ -54,7 +54,7 @@ using namespace ea;
 
 namespace {
 
-constexpr int MR_THREADS = 256;
+constexpr int MR_THREADS = 256, MR_BX = 128;  // blocks of 128 x 2 threads (the decode kernel's block width)
 constexpr int MR_NONE = -1200000000;  // reference exponent of a row without a visible key so far
 constexpr int MR_HEAD = 64;           // a weight may exceed the row's reference by 2^64 before it moves
 constexpr int MR_LIST = 64;
@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
     typedef MRowSmem<RS, DK, CPL> Smem;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     Smem& S = *reinterpret_cast<Smem*>(smem_raw);
-    const int tid = (int)threadIdx.x;
+    const int tid = (int)(threadIdx.x + MR_BX * threadIdx.y);
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int d = P.g.head_dim, dv = P.g.head_dim_v;
 
@@ -821,6 +821,6 @@ int ea::ea_launch_mrow(const Params& P, hipStream_t st) {
     Params Pc = P;
     void* args[] = {&Pc};
     const dim3 grid = P.dq_stream ? dim3((unsigned)P.dq_blocks) : dim3((unsigned)(P.nseg * P.nrb), (unsigned)P.nsplit);
-    e = hipLaunchKernel(mrow_fn_for(P), grid, dim3(MR_THREADS), args, mrow_lds_for(P), st);
+    e = hipLaunchKernel(mrow_fn_for(P), grid, dim3(MR_BX, MR_THREADS / MR_BX), args, mrow_lds_for(P), st);
     return e == hipSuccess ? 0 : -100 - (int)e;
 }

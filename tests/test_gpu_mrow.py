@@ -115,3 +115,16 @@ def test_equal_share_plan(gpu):
             assert st["decode_kernel_rows"] == flags.size and not flags.any(), st
             assert splits != 40 or st["decode_equal_share_steps"] == 1, st
             assert np.array_equal(got, want), st
+
+
+@pytest.mark.parametrize("splits", [0, 2, 3, 5])
+def test_combine_of_many_rows(gpu, splits):
+    """8192 rows, where the combine keeps 2 splits per load round instead of 8: one and two splits, and
+    more than fit a round, with empty splits on the causal rows; then 2 rows per segment of few
+    keys, on both sides of the line to the decode kernel."""
+    rng = np.random.default_rng(800 + splits)
+    prob = _rand_problem(rng, "normal", "normal", B=16, T=64, Hq=8, Hkv=2, S=330, d=64, dv=64)
+    _check(prob, default_alpha_bits(64), splits=splits)
+    for B, S in ((3, 500), (128, 128), (127, 128)):
+        prob = _rand_problem(rng, "normal", "outlier", B=B, T=1, Hq=32, Hkv=16, S=S, d=128, dv=128)
+        _check(prob, default_alpha_bits(128), splits=splits)
