@@ -326,6 +326,21 @@ class PagedKVCache:
                    "ea_hip_kv_digits_update")
 
 
+def _equal_runs(ql):
+    """The batch's runs of consecutive sequences with equal token counts, as (first, past the last)
+    pairs, where one launch per run beats one padded to the longest chunk, else None. A single run
+    needs no padding at all (4 x 5 tokens on 1000-key prefixes 197 -> 158 us a call, 300 tokens on
+    4000 keys 650 -> 625). Two or three pay for their extra launches when padding would more than
+    double the rows, to 512 or more: decode tokens padded to a prompt chunk's length run its
+    long serial blocks (150 tokens beside 11 decode tokens on 4000-key prefixes 937 -> 545 us, 64
+    beside 8 on 2000 399 -> 380); at 4 x 64 rows the two come out even (290, 302)."""
+    runs = [0] + [i for i in range(1, len(ql)) if ql[i] != ql[i - 1]] + [len(ql)]
+    n = len(runs) - 1
+    if n == 1 or (n <= 3 and len(ql) * max(ql) > 2 * sum(ql) and len(ql) * max(ql) >= 512):
+        return list(zip(runs[:-1], runs[1:]))
+    return None
+
+
 class ExactAttentionBackend:
     """Certified attention over a PagedKVCache. `alpha` is the base-2 logit scale as an fp32
     value; `alpha_bits=` passes its bit pattern instead."""
@@ -337,12 +352,13 @@ class ExactAttentionBackend:
         self._last = None  # the latest launch: its ea_* arguments and the tensors they point at
         self._geoms = {}   # ea_geometry per (B, T): only max_seq_len changes between launches
 
-    def _launch(self, seqs, qd, kvl, tree_mask=None, tree_base=None, digits_slot=None, staged=None, stream=None):
+    def _launch(self, seqs, qd, kvl, tree_mask=None, tree_base=None, digits_slot=None, staged=None, stream=None,
+                dst=None):
         """Enqueue one ea_hip_attention call over sequences `seqs` on torch's current stream.
         qd: (B, T, Hq, d) int16 device tensor, row (b, t, h) = token t of sequence seqs[b];
         kvl: (B*T,) int32 device tensor of visible prefix lengths; staged: the device seq_len and
-        block-table offset vectors of `seqs` when the caller uploaded them already. Returns device
-        (out, flags)."""
+        block-table offset vectors of `seqs` when the caller uploaded them already; dst: contiguous
+        (out, flags) to write. Returns device (out, flags)."""
         c = self.cache
         torch = c.torch
         lib = hip.load()
@@ -356,8 +372,11 @@ class ExactAttentionBackend:
             g["num_seqs"] = B
             gc = self._geoms[(B, T, Hq)] = hip.geometry(g)
         gc.max_seq_len = max(1, max(lens))
-        out = torch.empty((B, T, Hq, d), dtype=torch.int32 if self.out == "fp32" else torch.int16, device=c.dev)
-        flags = torch.empty(B * T * Hq, dtype=torch.uint8, device=c.dev)
+        if dst is not None:
+            out, flags = dst
+        else:
+            out = torch.empty((B, T, Hq, d), dtype=torch.int32 if self.out == "fp32" else torch.int16, device=c.dev)
+            flags = torch.empty(B * T * Hq, dtype=torch.uint8, device=c.dev)
         tm = tb = None
         if staged is not None:
             seq, off = staged[0], staged[1]
@@ -396,17 +415,17 @@ class ExactAttentionBackend:
         st = stream if stream is not None else hip._stream_ptr(torch)
         hip._check(lib.ea_hip_attention(ctypes.byref(gc), ctypes.byref(b), ctypes.byref(o), ws.data_ptr(), int(nb.value),
                                         st), "ea_hip_attention")
-        self._last = {"args": (gc, b, o), "keep": (qd, kvl, seq, off, tm, tb, staged), "out": out, "flags": flags,
+        self._last = {"args": (gc, b, o), "before": [], "keep": (qd, kvl, seq, off, tm, tb, staged), "out": out, "flags": flags,
                       "ret": None}
         return out, flags
 
     def _exact_tier(self) -> None:
-        """The host exact tier on the latest launch (ea_hip_exact_rows): waits for torch's current
+        """The host exact tier on the latest call's launches (ea_hip_exact_rows): waits for torch's current
         stream and recomputes every row left at flag 1 in place (flag 0, or 2 on a domain error)."""
         c = self.cache
-        gc, b, o = self._last["args"]
-        hip._check(hip.load().ea_hip_exact_rows(ctypes.byref(gc), ctypes.byref(b), ctypes.byref(o),
-                                                hip._stream_ptr(c.torch)), "ea_hip_exact_rows")
+        for gc, b, o in self._last["before"] + [self._last["args"]]:
+            hip._check(hip.load().ea_hip_exact_rows(ctypes.byref(gc), ctypes.byref(b), ctypes.byref(o),
+                                                    hip._stream_ptr(c.torch)), "ea_hip_exact_rows")
 
     def _run(self, seqs, q, kv_len, tree_mask=None, tree_base=None, digits_slot=None):
         """_launch, then the result on the host: (out bits (B, T, Hq, d), flags); flag 2 raises."""
@@ -455,19 +474,27 @@ class ExactAttentionBackend:
         plan = c._plan_append(seqs, ql, key, value, checked=True)
         lens = np.asarray([c.length[s] for s in seqs], dtype=np.int32)
         mine = [lens, np.asarray(seqs, dtype=np.int64) * c.max_pages, np.asarray(seqs, dtype=np.int32)]
+        plain = query.dim() == 3 and query.element_size() == 2 and query.device == c.k.device
+        runs = _equal_runs(ql) if T > 1 and plain else None
         if T > 1:
             start = np.concatenate([[0], np.cumsum(ql)])
             b_of = np.repeat(np.arange(B), ql)
             j_of = np.arange(ntok) - start[b_of]
-            kvl_h = np.zeros(B * T, dtype=np.int32)
-            kvl_h[b_of * T + j_of] = np.asarray(prefix)[b_of] + j_of + 1
-            mine += [kvl_h, (b_of * T + j_of).astype(np.int64)]
+            seen = (np.asarray(prefix)[b_of] + j_of + 1).astype(np.int32)
+            if runs is not None:
+                mine.append(seen)
+            else:
+                kvl_h = np.zeros(B * T, dtype=np.int32)
+                kvl_h[b_of * T + j_of] = seen
+                mine += [kvl_h, (b_of * T + j_of).astype(np.int64)]
         n_app = len(plan["arrays"])
         ts = torch.cuda.current_stream(c.dev)
         st = ctypes.c_void_p(ts.cuda_stream)
         dev = c.stage.put(*plan["arrays"], *mine, stream=ts)
         c._apply_append(plan, dev[:n_app], st)
         staged = (dev[n_app], dev[n_app + 1], dev[n_app + 2])
+        if runs is not None:
+            return self._forward_runs(query, list(seqs), ql, runs, staged, dev[n_app + 3], st)
         # one token per sequence sees the whole sequence: its visible length is the sequence's
         kvl = dev[n_app + 3] if T > 1 else dev[n_app]
         row = dev[n_app + 4] if T > 1 else None
@@ -486,6 +513,32 @@ class ExactAttentionBackend:
         else:
             ret = (out.view(B * T, Hq, -1).index_select(0, row), flags.view(B * T, Hq).index_select(0, row))
         self._last["ret"] = (ret, row, T)
+        return ret
+
+    def _forward_runs(self, query, seqs, ql, runs, staged, kvl, st):
+        """forward() over runs of consecutive sequences with equally many tokens: one launch each,
+        on the run's rows of the flattened query and output (no padding, gather or scatter).
+        staged, kvl: device vectors over all sequences and tokens. The query is copied, as the
+        padded path does: the exact tier may read it after the caller has reused its own."""
+        torch, dev = self.cache.torch, self.cache.dev
+        ntok, Hq, d = query.shape
+        q16 = query.view(torch.int16).clone(memory_format=torch.contiguous_format)
+        out = torch.empty((ntok, Hq, d), dtype=torch.int32 if self.out == "fp32" else torch.int16, device=dev)
+        flags = torch.empty((ntok, Hq), dtype=torch.uint8, device=dev)
+        before, keep, t0 = [], [], 0
+        for i0, i1 in runs:
+            B, T = i1 - i0, ql[i0]
+            t1 = t0 + B * T
+            if keep:
+                # a launch of the same shape changes the shared geometry's max_seq_len
+                gc, b, o = self._last["args"]
+                before.append((hip.Geometry.from_buffer_copy(gc), b, o))
+            self._launch(seqs[i0:i1], q16[t0:t1].view(B, T, Hq, d), kvl[t0:t1], digits_slot=seqs[0],
+                         staged=tuple(x[i0:i1] for x in staged), stream=st, dst=(out[t0:t1], flags[t0:t1]))
+            keep.append(self._last["keep"])
+            t0 = t1
+        ret = (out, flags)
+        self._last.update(before=before, keep=keep, out=out, flags=flags, ret=(ret, None, 1))
         return ret
 
     def check_flags(self, flags) -> None:
@@ -750,7 +803,9 @@ def hf_attention(module, query, key, value, attention_mask=None, scaling=None, d
     out = torch.empty((B, ql, H, D), dtype=torch.bfloat16, device=dev)
     flags = torch.empty(B * ql * H, dtype=torch.uint8, device=dev)
     lens = torch.full((B,), kl, dtype=torch.int32, device=dev)
-    kvl = (torch.arange(kl - ql + 1, kl + 1, dtype=torch.int32, device=dev)).repeat(B)
+    kvl = torch.arange(kl - ql + 1, kl + 1, dtype=torch.int32, device=dev)
+    if B > 1:
+        kvl = kvl.repeat(B)
     g = hip.geometry(dict(num_seqs=B, num_tokens=ql, num_q_heads=H, num_kv_heads=Hkv, head_dim=D, head_dim_v=D,
                           q_seq_stride=query.stride(0), q_tok_stride=query.stride(2), q_head_stride=query.stride(1),
                           o_seq_stride=ql * H * D, o_tok_stride=H * D, o_head_stride=D,
@@ -770,6 +825,8 @@ def hf_attention(module, query, key, value, attention_mask=None, scaling=None, d
                     out=out.data_ptr(), flags=flags.data_ptr())
     hip._check(lib.ea_hip_attention(ctypes.byref(g), ctypes.byref(b), ctypes.byref(o), ws.data_ptr(), int(nb.value),
                                     hip._stream_ptr(torch)), "ea_hip_attention")
+    if not bool(flags.any().item()):  # the usual case: one wait for the launch
+        return out, None
     if bool((flags == 1).any().item()):
         # rows the device tiers left uncertified: the host exact tier, in place
         hip._check(lib.ea_hip_exact_rows(ctypes.byref(g), ctypes.byref(b), ctypes.byref(o), hip._stream_ptr(torch)),

@@ -462,3 +462,47 @@ def test_kv_append_scatter(gpu, row_elems):
     assert np.array_equal(kpd.cpu().numpy().view(np.uint16), kp)
     assert np.array_equal(vpd.cpu().numpy().view(np.uint16), vp)
     assert np.array_equal(btd.cpu().numpy(), bt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,out", [(128, "bf16"), (64, "fp32")])
+def test_forward_runs_match_oracle(gpu, d, out):
+    """forward() on batches whose runs of equal token counts are launched one by one: one run, a
+    chunk after and between decode tokens (the outer runs share one shape but not their lengths),
+    and a batch that stays padded; query views off 16-byte alignment. Then the exact tier on every
+    row of every run, after the caller has overwritten its query, gives the same bits."""
+    import torch
+    from exactattention_amd.serving import ExactAttentionBackend, PagedKVCache, _equal_runs
+    rng = np.random.default_rng(91)
+    Hq, Hkv = 4, 2
+    ab = default_alpha_bits(d)
+    cache = PagedKVCache(num_pages=120, page_size=16, num_kv_heads=Hkv, head_dim=d, max_seqs=5, max_seq_len=512)
+    be = ExactAttentionBackend(cache, Hq, alpha_bits=ab, out=out)
+    slots = [cache.add_sequence() for _ in range(5)]
+    hist = {s: (np.zeros((0, Hkv, d), np.uint16), np.zeros((0, Hkv, d), np.uint16)) for s in slots}
+    for seqs, lens, runs in [([1, 0], [40, 40], 1), ([0, 2, 1, 3], [1, 1, 1, 130], 2),
+                             ([1, 3, 4, 0, 2], [1, 1, 120, 1, 1], 3), ([0, 3, 4, 1], [1, 70, 1, 69], 0),
+                             ([4], [5], 1)]:
+        assert len(_equal_runs(lens) or []) == runs
+        n = sum(lens)
+        q, k, v = bf16(rng, (n, Hq, d)), bf16(rng, (n, Hkv, d)), bf16(rng, (n, Hkv, d))
+        odd = torch.zeros(n * Hq * d + 1, dtype=torch.int16, device="cuda")[1:].view(n, Hq, d)
+        odd.copy_(torch.from_numpy(q.view(np.int16)))
+        o, fl = be.forward(odd, torch.from_numpy(k.view(np.int16)).cuda(), torch.from_numpy(v.view(np.int16)).cuda(),
+                           seqs, lens)
+        be.check_flags(fl)
+        want, at = [], 0
+        for s, T in zip(seqs, lens):
+            L = len(hist[s][0])
+            hist[s] = (np.concatenate([hist[s][0], k[at:at + T]]), np.concatenate([hist[s][1], v[at:at + T]]))
+            want.append(_oracle_rows(q[at:at + T], *hist[s], L + 1 + np.arange(T), ab, out=out))
+            at += T
+        want = np.concatenate(want)
+        assert o.shape == (n, Hq, d) and not fl.any().item()
+        assert np.array_equal(o.cpu().numpy().view(want.dtype), want), lens
+        if runs:
+            odd.zero_()
+            o.zero_()
+            fl.fill_(1)
+            be.check_flags(fl)
+            assert not fl.any().item() and np.array_equal(o.cpu().numpy().view(want.dtype), want), lens
