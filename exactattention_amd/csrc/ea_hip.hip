@@ -1,16 +1,18 @@
 // Certified split-KV ExactAttention for AMD Instinct MI355X (gfx950): kernels and C ABI.
 //
 // One step is four launches on the caller's stream, with fixed grids and no memsets:
-//   ea_prep      q rows -> fp64 + exponent ranges; clears the tier-2 work counter (the decode
-//                kernel on uniform splits does both itself, and the step is three launches)
+//   ea_prep      q rows -> fp64 + exponent ranges; clears the tier-2 work counter (ea_decode and
+//                ea_mrow on uniform splits do both themselves, and the step is three launches;
+//                ea_mrow's equal-share plan takes ea_plan here)
 //   ea_split     tier 1 (ea_decode, ea_mrow where they apply): per (segment, row block, KV split) an
 //                fp64 pass over 64-key tiles:
 //                exact scores (checked), certified logits and weights, P.V partials with
 //                rigorous error bounds. Writes one partial per (split, row).
 //   ea_combine   merges the split partials in the caller's order and certifies RN(N/Z) per
 //                channel; appends rows it cannot certify to the tier-2 work list
-//   ea_tier2     per listed row: 128-bit windowed scores, 128-bit exp2 enclosure, 128-bit
-//                fixed-point Z and N with counted truncation, exact final rounding
+//   ea_tier2     per listed row: a double-double pass with error bounds; for the rows it leaves,
+//                128-bit windowed scores, 128-bit exp2 enclosure, 128-bit fixed-point Z and N with
+//                counted truncation, exact final rounding
 // Reference behaviour: src/exactattn/triton_kernels.py:1324-1519 (split, combine, tier 2,
 // host fallback) and docs/SPEC.md (the definition the bits must equal).
 #include <hip/hip_runtime.h>
@@ -1305,7 +1307,7 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // rows ea_decode (whose 2-row blocks read at the rate of a large copy) takes the steps of 4096 or more
 // segment tiles, and this kernel, with half its tile latency (1.9 against 3.5 us) and splits down to
 // a tile, the shorter ones. 16/8 heads, the step's kernels, ea_decode -> here: 1 x 300 keys 36.6 ->
-// 17.2 us, 1 x 4K 39.8 -> 28, 16 x 1K 44.9 -> 40.4, 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134,
+// 17.2 us, 1 x 4K 39.8 -> 31, 16 x 1K 44.9 -> 40.4, 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134,
 // 32 x 4K 117 -> 131. Any other head size: always (ea_split takes what the pointers or pages do not
 // allow).
 int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {

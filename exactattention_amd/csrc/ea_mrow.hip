@@ -13,9 +13,9 @@
 // 25 per pair and lane for the certified weight.
 //
 // Measured against what ran before (MI355X, equal bits): 8 sequences of 16K keys, 16 rows, d = 128
-// 693 -> 220 us (ea_decode, 8 row blocks); 32 ragged sequences to 4K keys, 8 rows 228 -> 82 us;
+// 693 -> 226 us (ea_decode, 8 row blocks); 32 ragged sequences to 4K keys, 8 rows 228 -> 82 us;
 // 16 ragged sequences to 8K keys, 4 rows, d = 64 157 -> 41 us (ea_split); causal prefill of 2048
-// tokens, 32/8 heads, d = 64 2.89 -> 0.61 ms (ea_split). The VALU's own time is 162 of the 220 us
+// tokens, 32/8 heads, d = 64 2.89 -> 0.65 ms (ea_split). The VALU's own time is 162 of the 226 us
 // (16 rows), 102 of 143 us (8 rows, 32 x 4K keys) and 65 of 115 us (4 rows, bound by memory).
 //
 // The undecided pairs' exact path lives outside the step loop (a list in LDS, flush()): in it, its
