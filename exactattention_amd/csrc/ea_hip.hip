@@ -1101,8 +1101,7 @@ __device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last,
 
 // Tier 2: the listed rows in double-double (ea_refine.h), in EA_DD_PARTS key chunks in all when few
 // rows are listed; then, where a row stays undecided, the last block to finish takes what is left in
-// 128-bit arithmetic. force_tier2 sends every row straight to the 128-bit path, over EA_T2_BLOCKS
-// blocks. Measured: the 70 rows that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
+// 128-bit arithmetic. Measured: the 70 rows that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
 // 4096-key bf16 row after a prefill step 116 -> 35 us; an empty list 4.0-4.5 us
 // in the trace; 512 blocks cost a C2 step 1.8 us, so bf16 steps, which list few rows, launch 32.
 __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
@@ -1113,10 +1112,6 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
     __shared__ int s_last;
     const int cnt = *P.wl_cnt;
     if (cnt == 0) return;  // the usual case
-    if (P.t2_force) {
-        t2_rows(P, S.t2, s_last, cnt, cnt >= EA_T2_BLOCKS ? 1 : EA_T2_BLOCKS / cnt, (int)blockIdx.x, EA_T2_BLOCKS, false);
-        return;
-    }
     // every item of a split row is in flight at once (a block each, a partial each, a count per row)
     // and no chunk is shorter than a pass of 128 keys
     const int C = cnt <= EA_T2_ROWS ? min(min(EA_DD_PARTS, (int)gridDim.x) / cnt, (P.t2_keys + EA_DD_KEYS - 1) / EA_DD_KEYS) : 1;
@@ -1133,6 +1128,17 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
     __syncthreads();
     if (!s_last) return;
     t2_rows(P, S.t2, s_last, cnt, 1, 0, 1, true);
+}
+
+// force_tier2: every row straight to the 128-bit path, over EA_T2_BLOCKS blocks. A kernel of its own:
+// beside the double-double pass the body spills 413 SGPRs instead of 179 (32 rows of 32K keys 8.9 ms
+// against 6.9).
+__global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2_wide(Params P) {
+    __shared__ T2Smem S;
+    __shared__ int s_last;
+    const int cnt = *P.wl_cnt;
+    if (cnt > 0)
+        t2_rows(P, S, s_last, cnt, cnt >= EA_T2_BLOCKS ? 1 : EA_T2_BLOCKS / cnt, (int)blockIdx.x, EA_T2_BLOCKS, false);
 }
 
 // Lists every row for tier 2 (ea_options.force_tier2); runs after tier 1, so nothing else appends.
@@ -1598,7 +1604,6 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     P.t2M = (int32_t*)(ws + pl.off_t2M);
     P.t2E = (int64_t*)(ws + pl.off_t2E);
     P.ddpart = (void*)(ws + pl.off_t2E);
-    P.t2_force = o->force_tier2 ? 1 : 0;
     P.t2_keys = pl.t2_keys;
     P.pfq = (uint8_t*)(ws + pl.off_pfq);
     P.pfqm = (void*)(ws + pl.off_pfqm);
@@ -1674,7 +1679,10 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         if ((rc = mark(3))) return rc;
         if (o->tier2) {
             if ((rc = list_all(P, o, rb4 * 4 / 256 + 1, st))) return rc;
-            hipLaunchKernelGGL(ea_tier2, dim3(P.t2_force ? EA_T2_BLOCKS : EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
+            if (o->force_tier2)
+                hipLaunchKernelGGL(ea_tier2_wide, dim3(EA_T2_BLOCKS), dim3(EA_T2_THREADS), 0, st, P);
+            else
+                hipLaunchKernelGGL(ea_tier2, dim3(EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
             rc = herr(hipGetLastError());
             if (rc) return rc;
         }
@@ -1737,7 +1745,10 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     if ((rc = mark(3))) return rc;
     if (o->tier2) {
         if ((rc = list_all(P, o, rb4 * 4 / 256 + 1, st))) return rc;
-        hipLaunchKernelGGL(ea_tier2, dim3(P.t2_force ? EA_T2_BLOCKS : EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
+        if (o->force_tier2)
+            hipLaunchKernelGGL(ea_tier2_wide, dim3(EA_T2_BLOCKS), dim3(EA_T2_THREADS), 0, st, P);
+        else
+            hipLaunchKernelGGL(ea_tier2, dim3(EA_DD_BLOCKS(P.out_fp32)), dim3(EA_T2_THREADS), 0, st, P);
         rc = herr(hipGetLastError());
         if (rc) return rc;
     }

@@ -65,7 +65,6 @@ struct Params {
     int64_t* t2E;     // EA_T2_BLOCKS * max_keys
     void* ddpart;     // EA_DD_PARTS chunk partials of the double-double pass (DDPart, ea_refine.h)
     int32_t t2_keys;
-    int32_t t2_force;  // 1: every row is listed, straight for the 128-bit path
     // int8-MFMA prefill path (ea_prefill.hip)
     uint8_t* pfq;     // rows * 512: q digit planes
     void* pfqm;       // rows * sizeof(PfQMeta)
