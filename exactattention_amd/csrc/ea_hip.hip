@@ -1312,10 +1312,10 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // d = dv = 128: from 3 rows per segment on, up to where the int8 prefill kernel starts. With 1 or 2
 // rows ea_decode (whose 2-row blocks read at the rate of a large copy) takes the steps of 4096 or more
 // segment tiles, and this kernel, with half its tile latency (1.9 against 3.5 us) and splits down to
-// a tile, the shorter ones. 16/8 heads, the step's kernels, ea_decode -> here: 1 x 300 keys 36.6 ->
-// 17.2 us, 1 x 4K 39.8 -> 31, 16 x 1K 44.9 -> 40.4, 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134,
-// 32 x 4K 117 -> 131. Any other head size: always (ea_split takes what the pointers or pages do not
-// allow).
+// a tile, the shorter ones. 16/8 heads, graph replays of the step, ea_decode -> here: 1 x 600 keys 34.1
+// -> 16.2 us, 1 x 4K 35.1 -> 26.4, 1 x 16K 51.2 -> 38.6, 2 x 15000 66.7 -> 47.9, 16 x 1000 53.1 -> 38.6;
+// the step's kernels 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134, 32 x 4K 117 -> 131. Any other
+// head size: always (ea_split takes what the pointers or pages do not allow).
 int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {
     if (o->timers || o->kernel == EA_KERNEL_GENERAL) return 0;
     if (g->head_dim == 128 && g->head_dim_v == 128) {
@@ -1355,8 +1355,11 @@ void choose_splits(int64_t items, int maxlen, int splits, int* nsplit, int* spli
 }
 
 // The same for the multi-row kernel. First enough blocks to fill the device, down to one tile per
-// split (two from 16 splits on: merging 64 splits costs 16 us, 32 splits 10): a short context then
-// takes a step or two per wave instead of a chain of them. Then splits
+// split: a short context then takes a step or two per wave instead of a chain of them. A few long
+// segments stop earlier: a split costs the combine about what 4 tiles cost the kernel's chain, so the
+// count is kept near 2 sqrt(tiles) (one sequence, 16/8 heads, graph replays, at 16, 32, 64 and 128
+// splits: 8K keys 34.1, 31.6, 37.6, 44.3 us; 16K 47.1, 38.7, 43.5, 51.5; 30K 69, 49.9, 53, 61; 60K keys
+// on 4 KV heads 114, 73, 55.5, 65). Steps that fill the device take splits
 // of at most 512 keys, so that the equal-share plan (taken past one round of resident blocks) can
 // even out sequences of different lengths in shares of 8 tiles, while the partials stay below
 // MROW_PART and the workspace below the allocation-free entry point's array.
@@ -1368,8 +1371,9 @@ void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsp
         const int64_t items = pl.r_seg <= 8 ? (int64_t)pl.nseg * ((pl.r_seg + 1) / 2) : 2 * units;
         const int64_t rest = (int64_t)EA_T2_BLOCKS * 12 * maxlen + pl.rows * 1100;
         ns = 1;
-        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= (ns >= 8 ? 128 : 64)) ns *= 2;
-        while ((int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART &&
+        const int64_t tiles = ((int64_t)maxlen + EA_TILE - 1) / EA_TILE;
+        while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 64 && (int64_t)ns * ns <= 2 * tiles) ns *= 2;
+        while (items * ns >= 1024 && (int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART &&
                2 * ns * pl.rows * dv * 8 + rest <= MROW_WS)
             ns *= 2;
         while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
