@@ -32,10 +32,11 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
     const int J = (ns + 63) / 64;  // slabs of 64 splits: split 64 j + lane is this lane's in slab j
 
     // slab 0 may follow the caller's merge order: lane i holds split merge_order[i] when it is a
-    // permutation of [0, ns) (ns <= 64); the sums below come from wave reductions, and any
-    // summation order gives the same certified bits, so the order fixes only which lane loads what
+    // permutation of [0, ns) (the host passes it only where ns <= 64 is its length); the sums below
+    // come from wave reductions, and any summation order gives the same certified bits, so the order
+    // fixes only which lane loads what
     int si = lane;
-    bool mo_ok = P.merge_order != nullptr && ns <= 64 && !P.dq_stream;
+    bool mo_ok = P.merge_order != nullptr;
     if (mo_ok) {
         const int m = lane < ns ? P.merge_order[lane] : 0;
         const uint64_t bit = (lane < ns && m >= 0 && m < ns) ? (1ull << m) : 0ull;

@@ -1496,6 +1496,43 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
 
 int herr(hipError_t e) { return e == hipSuccess ? 0 : -100 - (int)e; }
 
+// The split count ea_hip_workspace_size reports, which ea_options.merge_order is a permutation of
+int reported_nsplit(const Plan& pl) { return pl.prefill ? pl.nsplit : pl.nsplit_gen; }
+
+// The caller's arrays and strides, as far as the choice of kernel and the split kernels read them
+void set_inputs(Params& P, const Plan& pl, const ea_geometry* g, const ea_buffers* bf) {
+    P.g = *g;
+    P.q = bf->q; P.k = bf->k; P.v = bf->v;
+    P.seq_len = bf->seq_len; P.kv_len = bf->kv_len; P.bt = bf->block_table; P.bt_off = bf->block_table_offset;
+    P.tree_mask = bf->tree_mask; P.tree_base = bf->tree_base;
+    P.nsplit = pl.nsplit; P.split_len = pl.split_len;
+    P.grp = pl.grp; P.r_seg = pl.r_seg; P.rb = pl.rb; P.nrb = pl.nrb; P.nseg = pl.nseg;
+    P.pshift = pl.pshift; P.dlog = pl.dlog; P.rows = pl.rows;
+}
+
+// The fp64 kernel of a step that does not take the prefill path (host logic): sets P.mrow, its row
+// blocks and its uniform splits. Returns whether it is ea_decode (false: ea_mrow or ea_split).
+bool choose_split_kernel(Params& P, const Plan& pl) {
+    P.nsplit = pl.nsplit_gen;
+    if (pl.mrow && pl.nseg > 0 && ea_mrow_eligible(P)) {
+        P.mrow = 1;
+    } else if (pl.mrow) {
+        P.rb = pl.gen_rb;
+        P.nrb = pl.gen_nrb;
+        P.split_len = pl.gen_split_len;
+        P.nsplit = pl.gen_nsplit;
+    }
+    return !P.mrow && pl.dq && pl.nseg > 0 && ea_decode_eligible(P);
+}
+
+// The caller's merge order where the combine may follow it: it has exactly the reported number of
+// entries, so never where the step merges another number of partials (a kernel that stands in for
+// ea_mrow has its own split count, the equal-share plan its own pieces), and the combine reads one
+// entry per lane. The order never changes a bit: it says which lane loads which partial.
+const int32_t* usable_merge_order(const Params& P, const Plan& pl, const ea_options* o) {
+    return (P.nsplit == reported_nsplit(pl) && P.nsplit <= 64 && !P.dq_stream) ? o->merge_order : nullptr;
+}
+
 }  // namespace
 
 // The allocation-free entry point's workspace (ea_hip_attention_noalloc): one array per device,
@@ -1547,7 +1584,27 @@ int ea_hip_workspace_size(const ea_geometry* g, const ea_options* o, size_t* byt
     int rc = make_plan(g, o, &pl);
     if (rc) return rc;
     if (bytes) *bytes = pl.total;
-    if (nsplit) *nsplit = pl.prefill ? pl.nsplit : pl.nsplit_gen;  // the decode kernel adds one partial slot
+    if (nsplit) *nsplit = reported_nsplit(pl);  // the equal-share plan adds one partial slot
+    return 0;
+}
+
+int ea_hip_step_route(const ea_geometry* g, const ea_buffers* bf, const ea_options* o, int32_t* kernel,
+                      int32_t* nsplit, int32_t* ordered) {
+    Plan pl;
+    int rc = make_plan(g, o, &pl);
+    if (rc) return rc;
+    if (!bf) return -1;
+    Params P;
+    memset(&P, 0, sizeof(P));
+    set_inputs(P, pl, g, bf);
+    int k = EA_KERNEL_PREFILL;
+    if (!pl.prefill) {
+        const bool decode = choose_split_kernel(P, pl);
+        k = P.mrow ? EA_ROUTE_MULTIROW : (decode ? EA_KERNEL_DECODE : EA_KERNEL_GENERAL);
+    }
+    if (kernel) *kernel = k;
+    if (nsplit) *nsplit = P.nsplit;
+    if (ordered) *ordered = !pl.prefill && usable_merge_order(P, pl, o) != nullptr;
     return 0;
 }
 
@@ -1573,11 +1630,8 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     if (((ab >> 23) & 0xFF) == 0xFF) return -3;
     Params P;
     memset(&P, 0, sizeof(P));
-    P.g = *g;
-    P.q = bf->q; P.k = bf->k; P.v = bf->v;
-    P.seq_len = bf->seq_len; P.kv_len = bf->kv_len; P.bt = bf->block_table; P.bt_off = bf->block_table_offset;
-    P.tree_mask = bf->tree_mask; P.tree_base = bf->tree_base;
-    P.out = bf->out; P.flags = bf->flags; P.stats = o->stats; P.merge_order = o->merge_order;
+    set_inputs(P, pl, g, bf);
+    P.out = bf->out; P.flags = bf->flags; P.stats = o->stats;
     P.timers = o->timers;
     float af;
     memcpy(&af, &ab, 4);
@@ -1590,9 +1644,6 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         P.ae = ex ? ex - 150 : -149;
     }
     P.out_fp32 = o->out_fp32 ? 1 : 0;
-    P.nsplit = pl.nsplit; P.split_len = pl.split_len;
-    P.grp = pl.grp; P.r_seg = pl.r_seg; P.rb = pl.rb; P.nrb = pl.nrb; P.nseg = pl.nseg;
-    P.pshift = pl.pshift; P.dlog = pl.dlog; P.rows = pl.rows;
     char* ws = (char*)workspace;
     P.q64 = (double*)(ws + pl.off_q64);
     P.qinfo = (int32_t*)(ws + pl.off_qinfo);
@@ -1630,19 +1681,11 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     P.dq_stream = 0;
     bool use_decode = false;
     if (!pl.prefill) {
-        int slots = 0, cus = 0, nsplit = pl.nsplit_gen;
-        if (pl.mrow && pl.nseg > 0 && ea_mrow_eligible(P)) {
-            P.mrow = 1;
-            if ((rc = ea_mrow_slots(P, &slots))) return rc;
-        } else if (pl.mrow) {
-            P.rb = pl.gen_rb;
-            P.nrb = pl.gen_nrb;
-            P.split_len = pl.gen_split_len;
-            nsplit = pl.gen_nsplit;
-        }
-        P.nsplit = nsplit;
-        use_decode = !P.mrow && pl.dq && pl.nseg > 0 && ea_decode_eligible(P);
+        int slots = 0, cus = 0;
+        use_decode = choose_split_kernel(P, pl);
+        if (P.mrow && (rc = ea_mrow_slots(P, &slots))) return rc;
         if (use_decode && (rc = ea_decode_slots(P, &slots, &cus))) return rc;
+        const int nsplit = P.nsplit;
         const int64_t units = (int64_t)P.nseg * P.nrb;
         // the equal-share plan when the uniform split grid would take more than one round of
         // resident blocks (long or ragged contexts); otherwise one block per (unit, split)
@@ -1667,6 +1710,7 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
             P.dq_rec_off = pl.dq_rec_off;
             P.dq_plan = (int32_t*)(ws + pl.off_dq);
         }
+        P.merge_order = usable_merge_order(P, pl, o);
     }
     auto mark = [&](int i) -> int {
         return (o->events && o->events[i]) ? herr(hipEventRecord((hipEvent_t)o->events[i], st)) : 0;

@@ -84,7 +84,11 @@ typedef struct ea_options {
     int32_t out_fp32;       /* 0 = bf16 output, 1 = fp32 output */
     int32_t splits;         /* KV splits per segment; 0 = choose for the device */
     int32_t tier2;          /* 1 = run the device tier 2 on rows tier 1 leaves uncertified */
-    const int32_t* merge_order; /* optional device permutation of [0, nsplit): combine order */
+    const int32_t* merge_order; /* optional device permutation of [0, nsplit), nsplit as
+                               ea_hip_workspace_size reports it: combine order. Followed where the
+                               step merges exactly nsplit <= 64 uniform splits (else unread: an
+                               equal-share plan, or a kernel that stands in for the multi-row one
+                               with splits of its own); never changes bits */
     int64_t* stats;         /* optional device int64[16], accumulated (+=):
                                [0] rows, [1] rows flagged by tier 1, [2] rows certified by tier 2,
                                [3] rows left flag 1, [4] rows flag 2, [5] tier-1 scores not
@@ -152,6 +156,16 @@ int ea_hip_workspace_size(const ea_geometry* g, const ea_options* o, size_t* byt
  * ea_hip_workspace_size. Reference counterpart: none (the reference slices the whole cache at
  * every launch, src/exactattn/triton_kernels.py:1255-1280). */
 int ea_hip_reads_kv_digits(const ea_geometry* g, const ea_options* o, int32_t* reads);
+
+/* Which tier-1 kernel ea_hip_attention would run for this geometry, these buffers and options
+ * (host logic only: pointers are looked at for their alignment, nothing is read): *kernel =
+ * EA_KERNEL_PREFILL, EA_KERNEL_DECODE (the d = 128 decode kernel), EA_KERNEL_GENERAL or
+ * EA_ROUTE_MULTIROW; *nsplit the KV splits that kernel takes (an equal-share plan, decided by the
+ * device's size, replaces them); *ordered = 1 when o->merge_order is followed on those splits. Each output may be NULL. Returns 0 or the
+ * negative codes of ea_hip_workspace_size, -1 for NULL buffers. No reference counterpart. */
+#define EA_ROUTE_MULTIROW 4
+int ea_hip_step_route(const ea_geometry* g, const ea_buffers* b, const ea_options* o, int32_t* kernel,
+                      int32_t* nsplit, int32_t* ordered);
 
 /* Enqueue one certified attention step on `stream`: q prep (inside the tier-1 kernel on the d =
  * 128 decode kernel's uniform grid), tier-1 split kernel, combine with

@@ -418,3 +418,43 @@ def test_kernel_choice_for_verification_segments():
     assert _reads_digits(geom(12, 1, 32768), fake) == (0, 1)     # 8 segments, 32K keys
     assert _reads_digits(geom(8, 32, 65536), fake) == (0, 0)     # 16 rows: decode at any length
     assert _reads_digits(geom(16, 1, 1024), fake) == (0, 1)      # 32 rows: always the int8 kernel
+
+
+def _step_geom(B, T, Hq, Hkv, d, S, dv=None, page=0):
+    """Geometry and stand-in pointers (never read) of a contiguous or NHD-paged step."""
+    dv = dv or d
+    npp = -(-S // page) if page else 0
+    ks, vs = ((page * Hkv * d, Hkv * d, d), (page * Hkv * dv, Hkv * dv, dv)) if page else ((Hkv * S * d, d, S * d),
+                                                                                         (Hkv * S * dv, dv, S * dv))
+    g = problem._geom(B, T, Hq, Hkv, d, dv, (T * Hq * d, Hq * d, d), (T * Hq * dv, Hq * dv, dv), ks, vs, page or 1,
+                      npp, S)
+    ptrs = {n: 1 << 20 for n in ("q", "k", "v", "seq_len", "kv_len", "out", "flags")}
+    if page:
+        ptrs["block_table"] = 1 << 20
+    return g, ptrs
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+def test_merge_order_is_read_only_at_its_own_length(d):
+    """merge_order holds exactly the split count ea_hip_workspace_size reports. Layouts the multi-row
+    kernel cannot read (pages of 8 keys, K or V rows off alignment) run a kernel with a split count of
+    its own: the combine then leaves the order alone instead of reading that many entries of it."""
+    from exactattention_amd import hip
+    other = 0
+    for B, T, grp, S in ((1, 1, 4, 16384), (1, 1, 1, 60000), (2, 3, 2, 5000), (4, 1, 8, 700), (1, 7, 1, 30000)):
+        for change in (dict(), dict(page=8), dict(page=16), dict(k=2), dict(v=2)):
+            g, ptrs = _step_geom(B, T, 8 * grp, 8, d, S, page=change.get("page", 0))
+            for n in ("k", "v"):
+                ptrs[n] += change.get(n, 0)
+            for splits in (0, 3, 40, 100):
+                rc, _, reported = _ws(g, splits)
+                kernel, ns, ordered = hip.step_route(g, ptrs, splits=splits, merge_order=1 << 20)
+                assert rc == 0 and (not ordered or (ns == reported and ns <= 64)), (change, S, splits, kernel, ns)
+                assert ordered or ns != reported or ns > 64, (change, S, splits, kernel, ns)
+                assert not hip.step_route(g, ptrs, splits=splits)[2]
+                other += ns != reported
+                if not change:
+                    assert kernel == ("decode" if d == 128 and grp * T <= 2 and B * 8 * -(-S // 64) >= 4096 else "multirow")
+                elif change.get("page") == 8 or "k" in change:
+                    assert kernel in ("decode", "general"), (change, kernel)
+    assert other > 0  # such steps exist: 32 against 64 splits of 16,384 keys
