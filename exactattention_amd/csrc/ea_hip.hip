@@ -1286,21 +1286,27 @@ __global__ void ea_kat_certify_quotient(int64_t n, const int64_t* v, int32_t fp3
 // ------------------------------------------------------------------------------------------------
 namespace {
 
+// One fp64 kernel's way to run tier 1: its row blocks per segment, its uniform KV splits, whether it
+// may take the equal-share plan (Params::dq_*; one more partial slot per unit), and its arrays in the
+// workspace
+struct Tier1 {
+    int rb, nrb, nsplit, split_len, dq;
+    size_t off_q64, off_qinfo, off_qn, off_pR, off_pn, off_pZ, off_pN, off_pV, end;
+};
+
 struct Plan {
-    int nsplit, split_len, rb, nrb, r_seg, grp, nseg, pshift, dlog;
+    int r_seg, grp, nseg, pshift, dlog;
     int64_t rows;
-    size_t off_q64, off_qinfo, off_qn, off_pR, off_pn, off_pZ, off_pN, off_pV, off_wl, off_cnt, off_t2M, off_t2E, total;
+    // mr: the multi-row kernel (ea_mrow.hip), where mrow is 1; gen: the decode or general kernel, for
+    // the other geometries and where the pointers do not suit the multi-row kernel. Only one of them
+    // runs, so their arrays share the memory
+    int mrow;
+    Tier1 mr, gen;
+    size_t off_front, off_wl, off_cnt, off_t2M, off_t2E, off_dd, total;
     size_t off_pfq, off_pfqm, off_pfkv, off_pfscr, off_pfpart, off_dq, off_t2part;
     int t2_keys;
     int prefill, pf_ntiles, pf_nrb, pf_nsplit, pf_tps;
-    // the decode kernel's equal-share decomposition (Params::dq_*): dq = 1 when the geometry may
-    // take it (the pointer checks come at launch); nsplit_gen = the uniform split count, nsplit =
-    // the partial slots per unit (one more for the pieces of the equal-share plan)
-    int dq, nsplit_gen, dq_units, dq_max_tiles, dq_rec_off;
-    // the multi-row kernel (ea_mrow.hip): its rows per block (0: not taken). Its row blocks per
-    // segment are rb and nrb, its splits nsplit_gen and split_len; gen_* are those of the kernel that
-    // runs when the pointers do not suit it (the same values where it is not taken)
-    int mrow, gen_rb, gen_nrb, gen_nsplit, gen_split_len;
+    int dq_units, dq_max_tiles, dq_rec_off;  // of the equal-share plan's array
 };
 
 // most blocks the decode kernel's equal-share decomposition launches (the plan array's size)
@@ -1362,23 +1368,72 @@ void choose_splits(int64_t items, int maxlen, int splits, int* nsplit, int* spli
 // on 4 KV heads 114, 73, 55.5, 65). Steps that fill the device take splits
 // of at most 512 keys, so that the equal-share plan (taken past one round of resident blocks) can
 // even out sequences of different lengths in shares of 8 tiles, while the partials stay below
-// MROW_PART and the workspace below the allocation-free entry point's array.
+// MROW_PART.
 void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsplit, int* split_len) {
     int ns = splits;
     if (ns == 0) {
-        const int64_t MROW_PART = 32 << 20, MROW_WS = 96 << 20;
-        const int64_t units = (int64_t)pl.nseg * pl.nrb;
+        const int64_t MROW_PART = 32 << 20;
+        const int64_t units = (int64_t)pl.nseg * pl.mr.nrb;
         const int64_t items = pl.r_seg <= 8 ? (int64_t)pl.nseg * ((pl.r_seg + 1) / 2) : 2 * units;
-        const int64_t rest = (int64_t)EA_T2_BLOCKS * 12 * maxlen + pl.rows * 1100;
-        ns = 1;
         const int64_t tiles = ((int64_t)maxlen + EA_TILE - 1) / EA_TILE;
+        ns = 1;
         while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 64 && (int64_t)ns * ns <= 2 * tiles) ns *= 2;
-        while (items * ns >= 1024 && (int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART &&
-               2 * ns * pl.rows * dv * 8 + rest <= MROW_WS)
-            ns *= 2;
+        while (items * ns >= 1024 && (int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART) ns *= 2;
         while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
     }
     split_tiles(maxlen, ns, nsplit, split_len);
+}
+
+// The workspace's layout for the plan's tier-1 choices, with the multi-row kernel's arrays or
+// without; returns its size. In turn: the tier-2 list and counters, tier 1's arrays, the 128-bit
+// path's, the prefill path's. When tier 2 runs, tier 1 and the prefill path are done with theirs, so
+// its double-double pass keeps its chunk partials there. They may reach into the 128-bit path's,
+// which starts after that pass.
+size_t lay_out(Plan* pl, const ea_geometry* g, const ea_options* o, bool mrow) {
+    const int64_t R = pl->rows;
+    const int dv = g->head_dim_v;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off = align_up(off + bytes);
+        return at;
+    };
+    pl->off_wl = take((size_t)(R > 0 ? R : 1) * 4);
+    pl->off_cnt = take(4 * EA_T2_CNT);
+    pl->off_front = off;
+    auto front = [&](Tier1& t, bool q) {
+        const size_t slots = (size_t)(t.nsplit + t.dq);
+        off = pl->off_front;
+        t.off_q64 = take(q ? (size_t)R * EA_MAXD * 8 : 0);
+        t.off_qinfo = take(q ? (size_t)R * 5 * 4 : 0);
+        t.off_qn = take(q ? (size_t)R * 4 * 8 : 0);
+        t.off_pR = take(slots * R * 4);
+        t.off_pn = take(slots * R * 4);
+        t.off_pZ = take(slots * R * 8);
+        t.off_pN = take(slots * R * dv * 8);
+        t.off_pV = take(slots * pl->nseg * t.nrb * dv * 4);
+        t.end = off;
+    };
+    front(pl->gen, true);
+    if (mrow) front(pl->mr, false);  // it converts its q rows itself
+    off = std::max(pl->gen.end, mrow ? pl->mr.end : 0);
+    pl->off_t2part = take(EA_T2_BLOCKS * sizeof(T2Part));
+    pl->dq_units = pl->nseg * std::max(pl->gen.dq ? pl->gen.nrb : 0, mrow && pl->mr.dq ? pl->mr.nrb : 0);
+    pl->dq_rec_off = (3 + pl->dq_units + 3) & ~3;  // 16-byte aligned block records after S
+    pl->off_dq = take(pl->dq_units > 0 ? (size_t)(pl->dq_rec_off + 4 * EA_DQ_MAX_BLOCKS) * 4 : 0);
+    pl->off_t2M = take((size_t)EA_T2_BLOCKS * pl->t2_keys * 4);
+    pl->off_t2E = take((size_t)EA_T2_BLOCKS * pl->t2_keys * 8);
+    pl->off_pfq = pl->off_pfqm = pl->off_pfkv = pl->off_pfscr = pl->off_pfpart = 0;
+    if (pl->prefill) {
+        pl->off_pfq = take((size_t)R * 512);
+        pl->off_pfqm = take((size_t)R * sizeof(PfQMeta));
+        // with a digit cache of the caller's there is nothing to slice into the workspace
+        if (!o->kv_digits) pl->off_pfkv = take((size_t)pl->nseg * pl->pf_ntiles * EA_PF_TILE_BYTES);
+        pl->off_pfscr = take((size_t)pl->nseg * pl->pf_nrb * pl->pf_nsplit * 512 * 32 * 8);
+        pl->off_pfpart = take(pl->pf_nsplit > 1 ? (size_t)pl->pf_nsplit * R * (sizeof(PfPart) + 128 * 16) : 0);
+    }
+    pl->off_dd = pl->off_front;
+    return pl->total = std::max(off, align_up(pl->off_dd + EA_DD_PARTS * sizeof(DDPart)));
 }
 
 int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
@@ -1394,20 +1449,6 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     if (o->prefill_waves != 0 && o->prefill_waves != 4 && o->prefill_waves != 8) return -2;
     pl->grp = g->num_q_heads / g->num_kv_heads;
     pl->r_seg = g->num_tokens * pl->grp;
-    // rows per block: the d = 128 decode kernel takes 1- or 2-row blocks (two waves per SIMD; a
-    // 4-row block needs more than 256 VGPRs, runs at one wave per SIMD and measured 4-14% slower
-    // on every multi-row shape: GQA 4 and 8 decode, 4-16 query tokens), the general split kernel
-    // 1, 2 or 4
-    const bool dec_rows = g->head_dim == 128 && g->head_dim_v == 128 && o->kernel != EA_KERNEL_GENERAL && !o->timers;
-    pl->rb = dec_rows ? std::min(pl->r_seg, 2) : (pl->r_seg >= 3 ? 4 : pl->r_seg);
-    pl->nrb = (pl->r_seg + pl->rb - 1) / pl->rb;
-    pl->gen_rb = pl->rb;
-    pl->gen_nrb = pl->nrb;
-    pl->mrow = mrow_rows(g, o, pl->r_seg);
-    if (pl->mrow) {
-        pl->rb = pl->mrow;
-        pl->nrb = (pl->r_seg + pl->rb - 1) / pl->rb;
-    }
     pl->nseg = g->num_seqs * g->num_kv_heads;
     pl->rows = (int64_t)g->num_seqs * g->num_tokens * g->num_q_heads;
     int ps = 0;
@@ -1416,60 +1457,14 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     int dl = 0;
     while ((1 << dl) < g->head_dim) ++dl;
     pl->dlog = dl;
-    int maxlen = g->max_seq_len > 0 ? g->max_seq_len : 1;
-    choose_splits(pl->nseg * (int64_t)pl->gen_nrb, maxlen, o->splits, &pl->gen_nsplit, &pl->gen_split_len);
-    pl->nsplit_gen = pl->gen_nsplit;
-    pl->split_len = pl->gen_split_len;
-    if (pl->mrow) choose_splits_mrow(*pl, maxlen, g->head_dim_v, o->splits, &pl->nsplit_gen, &pl->split_len);
-    // partial slots per unit, for whichever of the two kernels the pointers allow
-    pl->nsplit = std::max(pl->nsplit_gen, pl->gen_nsplit);
-    // the d = 128 decode kernel may run this step (ea_launch_decode also checks the pointers):
-    // its pieces need nsplit + 1 partial slots per unit
+    const int maxlen = g->max_seq_len > 0 ? g->max_seq_len : 1;
     const int64_t max_tiles = ((int64_t)maxlen + 63) / 64;
-    const int64_t max_nrb = std::max(pl->nrb, pl->gen_nrb);
-    int pf_nt = 0, pf_nr = 0;
-    pl->dq = (pl->mrow || (g->head_dim == 128 && g->head_dim_v == 128)) && o->kernel != EA_KERNEL_GENERAL &&
-             !o->timers && !ea_prefill_eligible(*g, pl->grp, o->kernel, &pf_nt, &pf_nr) && pl->rows < ((int64_t)1 << 30) &&
-             (int64_t)maxlen + 64 < ((int64_t)1 << 30) &&
-             (int64_t)pl->nseg * max_nrb * std::max<int64_t>(max_tiles, 1) < ((int64_t)1 << 30) &&
-             (int64_t)pl->nseg * max_nrb < ((int64_t)1 << 24);
-    pl->dq_units = (int)std::min<int64_t>(pl->nseg * max_nrb, 1 << 24);
     pl->dq_max_tiles = (int)max_tiles;
-    if (pl->dq) ++pl->nsplit;
-    int64_t R = pl->rows;
-    int dv = g->head_dim_v;
-    size_t off = 0;
-    pl->off_q64 = off; off = align_up(off + (size_t)R * EA_MAXD * 8);
-    pl->off_qinfo = off; off = align_up(off + (size_t)R * 5 * 4);
-    pl->off_qn = off; off = align_up(off + (size_t)R * 4 * 8);
-    pl->off_pR = off; off = align_up(off + (size_t)pl->nsplit * R * 4);
-    pl->off_pn = off; off = align_up(off + (size_t)pl->nsplit * R * 4);
-    pl->off_pZ = off; off = align_up(off + (size_t)pl->nsplit * R * 8);
-    pl->off_pN = off; off = align_up(off + (size_t)pl->nsplit * R * dv * 8);
-    pl->off_pV = off; off = align_up(off + (size_t)pl->nsplit * pl->nseg * std::max(pl->nrb, pl->gen_nrb) * dv * 4);
-    pl->off_wl = off; off = align_up(off + (size_t)(R > 0 ? R : 1) * 4);
-    pl->off_cnt = off; off = align_up(off + 4 * EA_T2_CNT);
-    pl->off_t2part = off; off = align_up(off + EA_T2_BLOCKS * sizeof(T2Part));
-    pl->off_dq = off;
-    pl->dq_rec_off = (3 + pl->dq_units + 3) & ~3;  // 16-byte aligned block records after S
-    if (pl->dq) off = align_up(off + (size_t)(pl->dq_rec_off + 4 * EA_DQ_MAX_BLOCKS) * 4);
-    pl->t2_keys = maxlen + 64;
-    pl->off_t2M = off; off = align_up(off + (size_t)EA_T2_BLOCKS * pl->t2_keys * 4);
-    // the double-double chunk partials share the 128-bit path's key scratch (never in use together)
-    pl->off_t2E = off;
-    off = align_up(off + std::max((size_t)EA_T2_BLOCKS * pl->t2_keys * 8, EA_DD_PARTS * sizeof(DDPart)));
+    pl->t2_keys = maxlen;  // a row's visible keys are distinct and below max_seq_len
     pl->prefill = ea_prefill_eligible(*g, pl->grp, o->kernel, &pl->pf_ntiles, &pl->pf_nrb) ? 1 : 0;
-    pl->off_pfq = pl->off_pfqm = pl->off_pfkv = pl->off_pfscr = pl->off_pfpart = 0;
     pl->pf_nsplit = pl->pf_tps = 1;
     if (pl->prefill) {
-        pl->off_pfq = off; off = align_up(off + (size_t)R * 512);
-        pl->off_pfqm = off; off = align_up(off + (size_t)R * sizeof(PfQMeta));
-        if (o->kv_digits) {
-            // the caller's digit cache holds the K/V tiles: nothing to slice into the workspace
-            if (o->kv_digits_tiles < pl->pf_ntiles) return -1;
-        } else {
-            pl->off_pfkv = off; off = align_up(off + (size_t)pl->nseg * pl->pf_ntiles * EA_PF_TILE_BYTES);
-        }
+        if (o->kv_digits && o->kv_digits_tiles < pl->pf_ntiles) return -1;
         // key splits when the (segment, row block) grid alone leaves CUs idle (one prefill block
         // fills a CU's LDS): double the splits while the grid is under 256 blocks and every split
         // keeps at least 16 tiles; a caller's split count is taken as given
@@ -1483,21 +1478,54 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
         if (pl->pf_tps < 1) pl->pf_tps = 1;
         pl->pf_nsplit = (pl->pf_ntiles + pl->pf_tps - 1) / pl->pf_tps;
         if (pl->pf_nsplit < 1) pl->pf_nsplit = 1;
-        pl->off_pfscr = off;
-        off = align_up(off + (size_t)pl->nseg * pl->pf_nrb * pl->pf_nsplit * 512 * 32 * 8);
-        pl->off_pfpart = off;
-        if (pl->pf_nsplit > 1)
-            off = align_up(off + (size_t)pl->pf_nsplit * R * (sizeof(PfPart) + 128 * 16));
-        pl->nsplit = pl->pf_nsplit;  // the split count this step uses
     }
-    pl->total = off;
+    // an equal-share plan over nrb row blocks per segment stays within its 30-bit arithmetic
+    auto dq_fits = [&](int64_t nrb) {
+        return o->kernel != EA_KERNEL_GENERAL && !o->timers && !pl->prefill && pl->rows < ((int64_t)1 << 30) &&
+               (int64_t)maxlen + 64 < ((int64_t)1 << 30) && pl->nseg * nrb * max_tiles < ((int64_t)1 << 30) &&
+               pl->nseg * nrb < ((int64_t)1 << 24);
+    };
+    // rows per block: the d = 128 decode kernel takes 1- or 2-row blocks (two waves per SIMD; a
+    // 4-row block needs more than 256 VGPRs, runs at one wave per SIMD and measured 4-14% slower
+    // on every multi-row shape: GQA 4 and 8 decode, 4-16 query tokens), the general split kernel
+    // 1, 2 or 4
+    Tier1& gen = pl->gen;
+    const bool d128 = g->head_dim == 128 && g->head_dim_v == 128;
+    const bool dec_rows = d128 && o->kernel != EA_KERNEL_GENERAL && !o->timers;
+    gen.rb = dec_rows ? std::min(pl->r_seg, 2) : (pl->r_seg >= 3 ? 4 : pl->r_seg);
+    gen.nrb = (pl->r_seg + gen.rb - 1) / gen.rb;
+    choose_splits(pl->nseg * (int64_t)gen.nrb, maxlen, o->splits, &gen.nsplit, &gen.split_len);
+    gen.dq = d128 && dq_fits(gen.nrb);
+    Tier1& mr = pl->mr;
+    mr.rb = mrow_rows(g, o, pl->r_seg);
+    pl->mrow = mr.rb > 0;
+    const size_t without = lay_out(pl, g, o, false);
+    if (!pl->mrow) return 0;
+    mr.nrb = (pl->r_seg + mr.rb - 1) / mr.rb;
+    choose_splits_mrow(*pl, maxlen, g->head_dim_v, o->splits, &mr.nsplit, &mr.split_len);
+    mr.dq = dq_fits(mr.nrb);
+    // A step that fits the allocation-free entry point's array with the other kernel's arrays fits it
+    // with this one's too: with fewer splits where the caller left them open, or without the
+    // equal-share plan. With as many partials as the other kernel and no plan it needs less: no q.
+    const size_t cap = EA_NOALLOC_SCRATCH_BYTES;
+    const Tier1 first = mr;
+    while (lay_out(pl, g, o, true) > cap && without <= cap) {
+        if (o->splits == 0 && mr.nsplit > 1) {
+            split_tiles(maxlen, mr.nsplit / 2, &mr.nsplit, &mr.split_len);
+        } else if (mr.dq) {
+            mr = first;
+            mr.dq = 0;
+        } else {
+            break;
+        }
+    }
     return 0;
 }
 
 int herr(hipError_t e) { return e == hipSuccess ? 0 : -100 - (int)e; }
 
 // The split count ea_hip_workspace_size reports, which ea_options.merge_order is a permutation of
-int reported_nsplit(const Plan& pl) { return pl.prefill ? pl.nsplit : pl.nsplit_gen; }
+int reported_nsplit(const Plan& pl) { return pl.prefill ? pl.pf_nsplit : (pl.mrow ? pl.mr.nsplit : pl.gen.nsplit); }
 
 // The caller's arrays and strides, as far as the choice of kernel and the split kernels read them
 void set_inputs(Params& P, const Plan& pl, const ea_geometry* g, const ea_buffers* bf) {
@@ -1505,24 +1533,20 @@ void set_inputs(Params& P, const Plan& pl, const ea_geometry* g, const ea_buffer
     P.q = bf->q; P.k = bf->k; P.v = bf->v;
     P.seq_len = bf->seq_len; P.kv_len = bf->kv_len; P.bt = bf->block_table; P.bt_off = bf->block_table_offset;
     P.tree_mask = bf->tree_mask; P.tree_base = bf->tree_base;
-    P.nsplit = pl.nsplit; P.split_len = pl.split_len;
-    P.grp = pl.grp; P.r_seg = pl.r_seg; P.rb = pl.rb; P.nrb = pl.nrb; P.nseg = pl.nseg;
+    P.grp = pl.grp; P.r_seg = pl.r_seg; P.nseg = pl.nseg;
     P.pshift = pl.pshift; P.dlog = pl.dlog; P.rows = pl.rows;
 }
 
 // The fp64 kernel of a step that does not take the prefill path (host logic): sets P.mrow, its row
 // blocks and its uniform splits. Returns whether it is ea_decode (false: ea_mrow or ea_split).
 bool choose_split_kernel(Params& P, const Plan& pl) {
-    P.nsplit = pl.nsplit_gen;
-    if (pl.mrow && pl.nseg > 0 && ea_mrow_eligible(P)) {
-        P.mrow = 1;
-    } else if (pl.mrow) {
-        P.rb = pl.gen_rb;
-        P.nrb = pl.gen_nrb;
-        P.split_len = pl.gen_split_len;
-        P.nsplit = pl.gen_nsplit;
-    }
-    return !P.mrow && pl.dq && pl.nseg > 0 && ea_decode_eligible(P);
+    P.mrow = pl.mrow && pl.nseg > 0 && ea_mrow_eligible(P);
+    const Tier1& t = P.mrow ? pl.mr : pl.gen;
+    P.rb = t.rb;
+    P.nrb = t.nrb;
+    P.nsplit = t.nsplit;
+    P.split_len = t.split_len;
+    return !P.mrow && t.dq && pl.nseg > 0 && ea_decode_eligible(P);
 }
 
 // The caller's merge order where the combine may follow it: it has exactly the reported number of
@@ -1603,7 +1627,7 @@ int ea_hip_step_route(const ea_geometry* g, const ea_buffers* bf, const ea_optio
         k = P.mrow ? EA_ROUTE_MULTIROW : (decode ? EA_KERNEL_DECODE : EA_KERNEL_GENERAL);
     }
     if (kernel) *kernel = k;
-    if (nsplit) *nsplit = P.nsplit;
+    if (nsplit) *nsplit = pl.prefill ? pl.pf_nsplit : P.nsplit;
     if (ordered) *ordered = !pl.prefill && usable_merge_order(P, pl, o) != nullptr;
     return 0;
 }
@@ -1645,20 +1669,12 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     }
     P.out_fp32 = o->out_fp32 ? 1 : 0;
     char* ws = (char*)workspace;
-    P.q64 = (double*)(ws + pl.off_q64);
-    P.qinfo = (int32_t*)(ws + pl.off_qinfo);
-    P.qn = (double*)(ws + pl.off_qn);
-    P.pR = (int32_t*)(ws + pl.off_pR);
-    P.pn = (int32_t*)(ws + pl.off_pn);
-    P.pZ = (double*)(ws + pl.off_pZ);
-    P.pN = (double*)(ws + pl.off_pN);
-    P.pV = (float*)(ws + pl.off_pV);
     P.wl = (int32_t*)(ws + pl.off_wl);
     P.wl_cnt = (int32_t*)(ws + pl.off_cnt);
     P.t2part = (void*)(ws + pl.off_t2part);
     P.t2M = (int32_t*)(ws + pl.off_t2M);
     P.t2E = (int64_t*)(ws + pl.off_t2E);
-    P.ddpart = (void*)(ws + pl.off_t2E);
+    P.ddpart = (void*)(ws + pl.off_dd);
     P.t2_keys = pl.t2_keys;
     P.pfq = (uint8_t*)(ws + pl.off_pfq);
     P.pfqm = (void*)(ws + pl.off_pfqm);
@@ -1699,7 +1715,8 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
             P.dq_lead = cus;
             P.pv_tiles = (int32_t)((5 * tt + den - 1) / den + 1);
         }
-        if ((use_decode || (P.mrow && pl.dq)) && units * nsplit > slots) {
+        const Tier1& t = P.mrow ? pl.mr : pl.gen;
+        if ((use_decode || P.mrow) && t.dq && units * nsplit > slots) {
             const int64_t nb = std::min<int64_t>(slots, EA_DQ_MAX_BLOCKS);
             P.dq_stream = 1;
             P.nsplit = nsplit + 1;
@@ -1711,6 +1728,14 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
             P.dq_plan = (int32_t*)(ws + pl.off_dq);
         }
         P.merge_order = usable_merge_order(P, pl, o);
+        P.q64 = (double*)(ws + t.off_q64);
+        P.qinfo = (int32_t*)(ws + t.off_qinfo);
+        P.qn = (double*)(ws + t.off_qn);
+        P.pR = (int32_t*)(ws + t.off_pR);
+        P.pn = (int32_t*)(ws + t.off_pn);
+        P.pZ = (double*)(ws + t.off_pZ);
+        P.pN = (double*)(ws + t.off_pN);
+        P.pV = (float*)(ws + t.off_pV);
     }
     auto mark = [&](int i) -> int {
         return (o->events && o->events[i]) ? herr(hipEventRecord((hipEvent_t)o->events[i], st)) : 0;

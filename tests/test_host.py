@@ -458,3 +458,37 @@ def test_merge_order_is_read_only_at_its_own_length(d):
                 elif change.get("page") == 8 or "k" in change:
                     assert kernel in ("decode", "general"), (change, kernel)
     assert other > 0  # such steps exist: 32 against 64 splits of 16,384 keys
+
+
+NOALLOC_BYTES = 128 << 20  # EA_NOALLOC_SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,d,S", [(1, 2048, 32, 8, 64, 2048), (1, 2048, 32, 8, 96, 2048),
+                                           (1, 512, 32, 8, 128, 2048), (16, 1, 16, 8, 128, 131072)])
+def test_steps_that_fit_the_allocation_free_array(B, T, Hq, Hkv, d, S):
+    """Causal prefill with 64- and 96-dim heads, a chunk on the int8 kernel and long-context decode stay
+    within the allocation-free entry point's array, with automatic splits and with one."""
+    for splits in (0, 1):
+        rc, nb, _ = _ws(_step_geom(B, T, Hq, Hkv, d, S)[0], splits)
+        assert rc == 0 and nb <= NOALLOC_BYTES, (splits, nb / 2 ** 20)
+
+
+def test_multi_row_steps_fit_where_the_general_kernel_fits():
+    """The multi-row kernel's partials never push a step past the allocation-free entry point's array
+    that the general kernel's arrays (its q in fp64 among them) leave inside it: sizes from small to
+    just under the limit, automatic and given split counts."""
+    rng = np.random.default_rng(3)
+    near = 0
+    for _ in range(6000):
+        d = int(rng.choice([8, 40, 64, 72, 96, 120]))
+        dv = d if rng.random() < 0.7 else int(rng.choice([2, 34, 64, 128]))
+        Hkv, grp = int(rng.choice([1, 2, 8])), int(rng.choice([1, 3, 4, 16]))
+        T, B = int(np.exp(rng.uniform(0, 8))), int(np.exp(rng.uniform(0, 5)))
+        S = max(T, int(np.exp(rng.uniform(3, 12.6))))
+        g = _step_geom(B, T, Hkv * grp, Hkv, d, S, dv)[0]
+        splits = int(rng.choice([0, 0, 1, 4, 50]))
+        nb = _ws(g, splits)[1]
+        want = _ws(g, splits, kernel=3)[1]
+        assert nb <= NOALLOC_BYTES or want > NOALLOC_BYTES, (B, T, Hkv, grp, d, dv, S, splits, nb, want)
+        near += NOALLOC_BYTES * 3 // 4 < want <= NOALLOC_BYTES
+    assert near > 50, near
