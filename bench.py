@@ -216,7 +216,8 @@ def published_shapes_line(steps: int, warmup: int) -> dict:
         st = dict(zip(STATS, dp.stats.cpu().numpy().tolist()))
         kv_bytes = 2 * B * Hkv * n * d * 2
         gbs = kv_bytes / (ms * 1e-3) / 1e9
-        kernel = "prefill" if st["prefill_kernel_rows"] else ("decode" if st["decode_kernel_rows"] else "general")
+        kernel = ("prefill" if st["prefill_kernel_rows"] else "multirow" if st["mrow_kernel_rows"] else
+                  "decode" if st["decode_kernel_rows"] else "general")
         out.append({"shape": f"{'decode' if T == 1 else 'verify T=8'} B={B} n={n}", "ms": round(ms, 5),
                     "kv_gbs": round(gbs, 1), "hbm_frac": round(gbs / HBM_PEAK_GBS, 4), "kernel": kernel,
                     "nsplit": dp.nsplit, "ref_ms_run1122": ref_ms, "ref_ms_best_run1124": ref_best,

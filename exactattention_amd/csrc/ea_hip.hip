@@ -1311,6 +1311,7 @@ struct Plan {
 
 // most blocks the decode kernel's equal-share decomposition launches (the plan array's size)
 #define EA_DQ_MAX_BLOCKS 4096
+#define EA_STATS 18  // ea_options.stats_entries of the callers whose stats go past 16
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -1325,6 +1326,7 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {
     if (o->timers || o->kernel == EA_KERNEL_GENERAL) return 0;
     if (g->head_dim == 128 && g->head_dim_v == 128) {
+        if (o->kernel == EA_KERNEL_DECODE) return 0;
         int nt = 0, nr = 0;
         const int64_t tiles = (int64_t)g->num_seqs * g->num_kv_heads * (((int64_t)g->max_seq_len + 63) / 64);
         if ((r_seg <= 2 && tiles >= 4096) ||
@@ -1656,6 +1658,7 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     memset(&P, 0, sizeof(P));
     set_inputs(P, pl, g, bf);
     P.out = bf->out; P.flags = bf->flags; P.stats = o->stats;
+    P.stats_x = o->stats && o->stats_entries == EA_STATS ? o->stats + 16 : nullptr;
     P.timers = o->timers;
     float af;
     memcpy(&af, &ab, 4);

@@ -54,7 +54,8 @@ using namespace ea;
 
 namespace {
 
-constexpr int MR_THREADS = 256, MR_BX = 128;  // blocks of 128 x 2 threads (the decode kernel's block width)
+// 128 x 2 threads: whoever looks for a captured step's fp64 tier-1 node knows it by that width
+constexpr int MR_THREADS = 256, MR_BX = 128;
 constexpr int MR_NONE = -1200000000;  // reference exponent of a row without a visible key so far
 constexpr int MR_HEAD = 64;           // a weight may exceed the row's reference by 2^64 before it moves
 constexpr int MR_LIST = 64;
@@ -131,6 +132,7 @@ __global__ void __launch_bounds__(MR_THREADS, (mr_waves<RS, DK>())) ea_mrow(Para
         // on uniform splits the step's first kernel clears the tier-2 work list and chunk counts
         if (!P.dq_stream && tid < EA_T2_CNT) P.wl_cnt[tid] = 0;
         if (tid == 0 && P.stats) atomicAdd((unsigned long long*)&P.stats[9], (unsigned long long)P.rows);
+        if (tid == 0 && P.stats_x) atomicAdd((unsigned long long*)&P.stats_x[0], (unsigned long long)P.rows);
     }
 
     // One piece: keys [kA, kB) of unit `item` (segment, row block), clipped to the unit's visible

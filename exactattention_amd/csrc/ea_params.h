@@ -39,6 +39,7 @@ struct Params {
     void* out;
     uint8_t* flags;
     int64_t* stats;
+    int64_t* stats_x;  // stats + 16 where the caller's array has those entries
     int64_t* timers;
     const int32_t* merge_order;
     double alpha;

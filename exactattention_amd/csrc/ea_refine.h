@@ -407,6 +407,7 @@ __device__ inline void dd_rows(const Params& P, DDSmem& S, int cnt, int C, DDPar
             if (tid == 0) {
                 atomicOr(&P.wl[slot], (int)0x80000000);  // left for the 128-bit path
                 atomicAdd(&P.wl_cnt[EA_T2_LEFT], 1);
+                if (P.stats_x) atomicAdd((unsigned long long*)&P.stats_x[1], 1ull);
             }
             continue;
         }

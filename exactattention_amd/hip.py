@@ -43,7 +43,7 @@ class Options(ctypes.Structure):
                 ("tier2", ctypes.c_int32), ("merge_order", P), ("stats", P), ("events", P), ("timers", P),
                 ("kv_digits", P), ("kv_digits_tiles", ctypes.c_int32), ("pad1", ctypes.c_int32),
                 ("kv_digits_slot", P), ("force_tier2", ctypes.c_int32), ("kernel", ctypes.c_int32),
-                ("prefill_waves", ctypes.c_int32), ("pad2", ctypes.c_int32)]
+                ("prefill_waves", ctypes.c_int32), ("stats_entries", ctypes.c_int32)]
 
 
 # ea_options.kernel (include/exactattn_hip.h EA_KERNEL_*)
@@ -55,7 +55,8 @@ EA_PF_TILE_BYTES = 69632  # one 64-key digit tile (ea_params.h)
 STATS = ["rows", "tier1_flagged", "tier2_certified", "uncertified", "domain_errors", "uncertified_scores",
          "undecided_weights", "uncertified_final", "slow_path_scores",
          "decode_kernel_rows", "prefill_kernel_rows", "prefill_epoch_folds", "prefill_cold_waves",
-         "host_exact_rows", "host_exact_refused", "decode_equal_share_steps"]
+         "host_exact_rows", "host_exact_refused", "decode_equal_share_steps", "mrow_kernel_rows",
+         "tier2_wide_rows"]
 
 
 def available() -> bool:
@@ -197,7 +198,7 @@ class DeviceProblem:
         nb, self.nsplit = workspace_size(self.geom, splits, self.out_fp32, self.kernel)
         self.workspace = torch.empty(max(nb, 256), dtype=torch.uint8, device=dev)
         self.ws_bytes = nb
-        self.stats = torch.zeros(16, dtype=torch.int64, device=dev)
+        self.stats = torch.zeros(len(STATS), dtype=torch.int64, device=dev)
         self._geom_c = geometry(self.geom)
 
     def buffers(self) -> Buffers:
@@ -218,7 +219,8 @@ def options(dp: "DeviceProblem", alpha_bits: int, merge_order=None, tier2: bool 
                    timers=None if timers is None else timers.data_ptr(),
                    kv_digits=None if kv_digits is None else kv_digits.buf.data_ptr(),
                    kv_digits_tiles=0 if kv_digits is None else kv_digits.tiles,
-                   force_tier2=int(force_tier2), kernel=dp.kernel, prefill_waves=dp.prefill_waves)
+                   force_tier2=int(force_tier2), kernel=dp.kernel, prefill_waves=dp.prefill_waves,
+                   stats_entries=len(STATS))
 
 
 def launch_hip(dp: DeviceProblem, alpha_bits: int, merge_order=None, tier2: bool = True, events=None,

@@ -95,14 +95,16 @@ typedef struct ea_options {
                                certified, [6] tier-1 weights not certified, [7] tier-1 final
                                roundings not certified, [8] scores taken by the per-pair exact
                                path, [9] rows whose tier 1 ran in the d = 128 decode
-                               kernel or the multi-row kernel (3 to 31 rows per
-                               sequence and KV head, and head sizes other than 128), [10] rows whose tier 1 ran in the int8-MFMA
-                               prefill kernel, [11] prefill epoch folds before the last
+                               kernel or the multi-row kernel, [10] rows whose tier 1
+                               ran in the int8-MFMA prefill kernel, [11] prefill epoch folds before the last
                                tile (waves), [12] prefill waves that ran the exact
                                per-pair path, [13] rows certified by the host exact
                                tier (ea_hip_exact_rows), [14] rows it refused (spread
                                limit, flag 2), [15] steps whose decode kernel ran
-                               the equal-share plan (either kernel) */
+                               the equal-share plan (either kernel). With stats_entries
+                               = 18, int64[18]: [16] the rows of [9] that the multi-row
+                               kernel took, [17] the rows that tier 2's double-double pass
+                               left to its 128-bit path */
     void* const* events;    /* optional: 5 hipEvent_t recorded on `stream` before prep (the
                                int8 path: q and K/V slicing; none on the decode kernel's uniform
                                grid, whose kernel converts q), the tier-1 kernel, the combine (the
@@ -130,10 +132,12 @@ typedef struct ea_options {
                                exact tier on whole problems; needs tier2 = 1) */
     int32_t kernel;         /* tier-1 kernel: EA_KERNEL_AUTO (by geometry), EA_KERNEL_PREFILL (the
                                int8 prefill kernel for every d = dv = 128 problem),
-                               EA_KERNEL_DECODE (never the prefill kernel), EA_KERNEL_GENERAL (the
-                               general fp64 split kernel for every problem); never changes bits */
+                               EA_KERNEL_DECODE (the decode kernel for every d = dv = 128 problem
+                               whose layout it reads; never the prefill kernel), EA_KERNEL_GENERAL
+                               (the general fp64 split kernel for every problem); never changes
+                               bits */
     int32_t prefill_waves;  /* prefill block shape: 0 or 8 = 8 waves, 4 = 4 waves (same bits) */
-    int32_t pad2;
+    int32_t stats_entries;  /* 18: stats has 18 entries; any other value: 16 */
 } ea_options;
 
 #define EA_KERNEL_AUTO 0

@@ -81,10 +81,11 @@ def test_prefill_step_in_a_graph(gpu):
         assert np.array_equal(o, want)
 
 
-def test_decode_kernel_repeats_back_to_back(gpu):
+@pytest.mark.parametrize("kernel", ["auto", "decode"])
+def test_decode_kernel_repeats_back_to_back(gpu, kernel):
     """bench.py times the decode kernel alone, relaunched with the captured step's parameters: the
     step holds exactly one such node, every repeat runs the decode kernel (its row counter moves by
-    the rows once per launch), and the repeats rewrite the workspace with the same bytes."""
+    the rows once per launch; the multi-row kernel in its place on a short step), and the repeats rewrite the workspace with the same bytes."""
     import sys
     import torch
     sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
@@ -98,13 +99,14 @@ def test_decode_kernel_repeats_back_to_back(gpu):
     seq = np.array([700, 513, 64, 1])
     prob = problem.to_paged(problem.contiguous(q, k, v, seq.reshape(B, 1), seq_len=seq), 16, rng, "NHD")
     ab = default_alpha_bits(d)
-    dp = DeviceProblem(prob, "bf16", 0, "cuda:0")
+    dp = DeviceProblem(prob, "bf16", 0, "cuda:0", kernel)
     launch_hip(dp, ab)
     torch.cuda.synchronize()
     out0 = dp.out.cpu().numpy().copy()
     ws0 = dp.workspace.cpu().numpy().copy()
     st0 = dict(zip(STATS, dp.stats.cpu().numpy().tolist()))
     assert st0["decode_kernel_rows"] == B * Hq
+    assert st0["mrow_kernel_rows"] == (B * Hq if kernel == "auto" else 0)
     reps = 3
     ms = bench.back_to_back_ms(dp, ab, 128, reps)
     torch.cuda.synchronize()

@@ -13,10 +13,10 @@ from test_gpu_parity import _oracle, _rand_problem, _run
 pytestmark = pytest.mark.gpu
 
 
-def _check(prob, ab, out="bf16", splits=0):
+def _check(prob, ab, out="bf16", splits=0, mrow=True):
     want, wflags = _oracle(prob, ab, out)
     got, flags, st = _run(prob, ab, out, splits)
-    assert st["decode_kernel_rows"] == flags.size, st
+    assert st["decode_kernel_rows"] == flags.size and st["mrow_kernel_rows"] == (flags.size if mrow else 0), st
     assert not flags.any() and not np.any(wflags), st
     assert np.array_equal(got, want), st
     return st
@@ -48,7 +48,7 @@ def test_value_kinds(gpu, rows, kind):
         ab = default_alpha_bits(d) if alpha is None else int(alpha.view(np.uint32))
         want, wflags = _oracle(prob, ab)
         got, flags, st = _run(prob, ab)
-        assert st["decode_kernel_rows"] == flags.size, st
+        assert st["mrow_kernel_rows"] == flags.size, st
         ok = flags.reshape(want.shape[:3]) == 0  # what the device tiers leave is the host tier's
         assert np.array_equal(got[ok], want[ok]) and (flags != 2).all(), st
 
@@ -112,7 +112,7 @@ def test_equal_share_plan(gpu):
         want, _ = _oracle(prob, ab)
         for splits in (0, 40, 1):
             got, flags, st = _run(prob, ab, splits=splits)
-            assert st["decode_kernel_rows"] == flags.size and not flags.any(), st
+            assert st["mrow_kernel_rows"] == flags.size and not flags.any(), st
             assert splits != 40 or st["decode_equal_share_steps"] == 1, st
             assert np.array_equal(got, want), st
 
@@ -127,4 +127,4 @@ def test_combine_of_many_rows(gpu, splits):
     _check(prob, default_alpha_bits(64), splits=splits)
     for B, S in ((3, 500), (128, 128), (127, 128)):
         prob = _rand_problem(rng, "normal", "outlier", B=B, T=1, Hq=32, Hkv=16, S=S, d=128, dv=128)
-        _check(prob, default_alpha_bits(128), splits=splits)
+        _check(prob, default_alpha_bits(128), splits=splits, mrow=B != 128)  # 128 x 16 x 2 tiles: ea_decode's

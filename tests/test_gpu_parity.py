@@ -25,6 +25,13 @@ def _run(prob, alpha_bits, out="bf16", splits=0, merge_order=None, **kw):
     return attention_problem(prob, None, out, splits, merge_order, True, False, alpha_bits=alpha_bits, **kw)
 
 
+def _run_decode(prob, alpha_bits, out="bf16", splits=0, **kw):
+    """_run on the d = 128 decode kernel, also where the automatic choice is the multi-row kernel."""
+    got, flags, st = _run(prob, alpha_bits, out, splits, kernel="decode", **kw)
+    assert st["decode_kernel_rows"] == flags.size and st["mrow_kernel_rows"] == 0, st
+    return got, flags, st
+
+
 def _oracle(prob, alpha_bits, out="bf16"):
     from oracle import oracle
     return oracle.attention_geom(prob, alpha_bits, out)
@@ -430,8 +437,8 @@ def test_decode_kernel_kinds_match_oracle(gpu, kind, vkind):
     prob = _rand_problem(rng, kind, vkind, B=2, T=1, Hq=4, Hkv=2, S=300, d=128, dv=128, causal=False)
     ab = default_alpha_bits(128)
     want, _ = _oracle(prob, ab)
-    for splits in (1, 3):
-        got, flags, st = _run(prob, ab, splits=splits)
+    for splits, run in ((1, _run), (3, _run), (1, _run_decode), (3, _run_decode)):
+        got, flags, st = run(prob, ab, splits=splits)
         assert st["decode_kernel_rows"] == prob["q"].shape[0] * prob["q"].shape[2], st
         assert not np.any(flags == 1), (splits, flags, st)
         assert np.array_equal(got, want), (splits, st)
@@ -454,14 +461,15 @@ def test_decode_kernel_shapes_pages_ragged(gpu, hq, hkv, T, ps):
         prob = problem.to_paged(prob, ps, np.random.default_rng(ps), "NHD")
     ab = default_alpha_bits(d)
     want, _ = _oracle(prob, ab)
-    for splits in (1, 2):
-        got, flags, st = _run(prob, ab, splits=splits)
+    for splits, run in ((1, _run), (2, _run), (1, _run_decode), (2, _run_decode)):
+        got, flags, st = run(prob, ab, splits=splits)
         assert st["decode_kernel_rows"] > 0, st
         assert not np.any(flags), (splits, st)
         assert np.array_equal(got, want), (splits, st)
 
 
-def test_decode_kernel_nonfinite_flags_exactly_the_rows_that_see_them(gpu):
+@pytest.mark.parametrize("run", [_run, _run_decode])
+def test_decode_kernel_nonfinite_flags_exactly_the_rows_that_see_them(gpu, run):
     rng = np.random.default_rng(44)
     prob = _rand_problem(rng, "normal", "normal", B=1, T=8, Hq=2, Hkv=1, S=200, d=128, dv=128)
     prob["seq_len"][:] = 200
@@ -469,7 +477,7 @@ def test_decode_kernel_nonfinite_flags_exactly_the_rows_that_see_them(gpu):
     prob["k"][0, 0, 140, 3] = 0x7FC0   # NaN key at position 140
     prob["v"][0, 0, 162, 100] = 0xFF80  # -inf value at position 162
     ab = default_alpha_bits(128)
-    got, flags, st = _run(prob, ab)
+    got, flags, st = run(prob, ab)
     assert st["decode_kernel_rows"] > 0, st
     kvl = prob["kv_len"]
     clean = {**prob, "k": prob["k"].copy(), "v": prob["v"].copy()}
@@ -484,8 +492,9 @@ def test_decode_kernel_nonfinite_flags_exactly_the_rows_that_see_them(gpu):
                 assert np.array_equal(got[0, t, h], want[0, t, h]), (t, h)
 
 
+@pytest.mark.parametrize("run", [_run, _run_decode])
 @pytest.mark.parametrize("splits", [1, 2, 4])
-def test_decode_kernel_converts_q_rows_itself(gpu, splits):
+def test_decode_kernel_converts_q_rows_itself(gpu, splits, run):
     """On the uniform grid the decode kernel converts its blocks' q rows (no prep launch): a NaN q
     row alone in the last, partial 2-row block of a segment (3 rows per segment), a -inf element
     in the first row of another block, and a q row of zeros, with 1, 2 and 4 splits writing the
@@ -503,7 +512,7 @@ def test_decode_kernel_converts_q_rows_itself(gpu, splits):
         clean["q"][b, t, h, :] = 0
     ab = default_alpha_bits(128)
     want, _ = _oracle(clean, ab)
-    got, flags, st = _run(prob, ab, splits=splits)
+    got, flags, st = run(prob, ab, splits=splits)
     assert st["decode_kernel_rows"] > 0 and st["decode_equal_share_steps"] == 0, st
     fl = flags.reshape(B, T, H)
     for b in range(B):
@@ -515,7 +524,7 @@ def test_decode_kernel_converts_q_rows_itself(gpu, splits):
                     assert fl[b, t, h] == 0, (b, t, h, flags)
                     assert np.array_equal(got[b, t, h], want[b, t, h]), (b, t, h)
     # the clean problem on the same geometry: no flag survives from the previous q rows
-    got2, flags2, _ = _run(clean, ab, splits=splits)
+    got2, flags2, _ = run(clean, ab, splits=splits)
     assert not np.any(flags2)
     assert np.array_equal(got2, want)
 
@@ -539,8 +548,9 @@ def test_decode_lead_wave_splits(gpu, B, S):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("run", [_run, _run_decode])
 @pytest.mark.parametrize("seed", range(401, 409))
-def test_decode_lead_wave_random_grids(gpu, seed):
+def test_decode_lead_wave_random_grids(gpu, seed, run):
     """Seeded random uniform decode grids of exactly 1,024 blocks (the weighted first wave on
     MI355X): GQA group 1-4 (2-row blocks, several per segment, the XCD permutation when the
     segment count is a multiple of 8), 1-2 tokens, ragged lengths, contiguous or paged NHD caches.
@@ -564,12 +574,12 @@ def test_decode_lead_wave_random_grids(gpu, seed):
         prob = problem.to_paged(prob, int(rng.choice([16, 64])), np.random.default_rng(seed), "NHD")
     ab = default_alpha_bits(128)
     want, _ = _oracle(prob, ab)
-    got, flags, st = _run(prob, ab)
+    got, flags, st = run(prob, ab)
     assert st["decode_kernel_rows"] > 0 and st["decode_equal_share_steps"] == 0, (seed, st)
     assert st["nsplit"] == ns, (seed, ns, st)
     assert not np.any(flags), (seed, st)
     assert np.array_equal(got, want), seed
-    got1, _, _ = _run(prob, ab, splits=1)
+    got1, _, _ = run(prob, ab, splits=1)
     assert np.array_equal(got1, want), seed
 
 
@@ -986,8 +996,9 @@ def test_decode_equal_share_plan(gpu, case):
     assert np.array_equal(got2, want) and not flags2.any()
 
 
+@pytest.mark.parametrize("run", [_run, _run_decode])
 @pytest.mark.parametrize("case", ["uniform", "equal_share"])
-def test_decode_xcd_placement(gpu, case):
+def test_decode_xcd_placement(gpu, case, run):
     """GQA 4 decode (2-row blocks, 2 units per segment, segments a multiple of 8): the decode
     kernel places a segment's row blocks on one XCD, on the uniform split grid and, with more
     units than an eighth of the equal-share plan's blocks, by a permutation of the shares. The
@@ -1006,7 +1017,7 @@ def test_decode_xcd_placement(gpu, case):
     v = bf16(rng, (B, Hkv, S, 128))
     base = problem.contiguous(q, k, v, lens.reshape(B, 1), seq_len=lens)
     prob = problem.to_paged(base, page, rng, "NHD")
-    got, flags, st = _run(prob, ab)
+    got, flags, st = run(prob, ab)
     assert st["decode_kernel_rows"] > 0 and not flags.any(), st
     assert st["decode_equal_share_steps"] == (1 if case == "equal_share" else 0), st
     ref, flags2, st2 = _run(prob, ab, kernel="general")
@@ -1017,8 +1028,9 @@ def test_decode_xcd_placement(gpu, case):
         assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("run", [_run, _run_decode])
 @pytest.mark.parametrize("seed", [301, 302, 303, 304, 305, 306])
-def test_decode_placement_random_many_segments(gpu, seed):
+def test_decode_placement_random_many_segments(gpu, seed, run):
     """Seeded geometries with 128-256 segments (8 KV heads) and 2-8 row blocks per segment, ragged
     lengths, pages of 16 or 64 keys, 1 or 2 tokens: the decode kernel, its row blocks placed by
     XCD on the uniform grid or the equal-share plan (whichever the step takes), gives the general
@@ -1037,7 +1049,7 @@ def test_decode_placement_random_many_segments(gpu, seed):
     v = bf16(rng, (B, Hkv, S, 128))
     base = problem.contiguous(q, k, v, kv, seq_len=lens)
     prob = problem.to_paged(base, int(rng.choice([16, 64])), rng, "NHD")
-    got, flags, st = _run(prob, ab)
+    got, flags, st = run(prob, ab)
     desc = f"seed {seed}: B={B} T={T} grp={grp} S={S} {st}"
     assert st["decode_kernel_rows"] > 0 and not flags.any(), desc
     ref, flags2, st2 = _run(prob, ab, kernel="general")

@@ -7,7 +7,7 @@ what is checked), head dims, GQA group, tokens per sequence, ragged sequence len
 causal / tree masks (tree keys overlapping the prefix and running past seq_len), input kinds, page
 size and layout, split count and output format. Every case must return the oracle's bits with
 every row certified by the device tiers or the host exact tier (fallback=True), and the sweep as a
-whole must have run each of the three tier-1 kernels.
+whole must have run each of the four tier-1 kernels.
 """
 
 import os
@@ -110,7 +110,7 @@ def _case(i):
 def test_random_geometries_match_oracle(gpu):
     from exactattention_amd.hip import attention_problem
     from oracle import exact, oracle
-    ran = {"decode": 0, "prefill": 0, "general": 0}
+    ran = {"decode": 0, "multirow": 0, "prefill": 0, "general": 0}
     for i in range(FIRST, FIRST + NCASES):
         prob, kernel, d, out, splits, desc = _case(i)
         ab = default_alpha_bits(d)
@@ -126,7 +126,9 @@ def test_random_geometries_match_oracle(gpu):
         got, flags, st = attention_problem(prob, None, out, splits, None, True, True, kernel=kernel, alpha_bits=ab)
         assert not np.any(flags), (desc, st)
         assert np.array_equal(got, want), (desc, st)
-        if st["decode_kernel_rows"]:
+        if st["mrow_kernel_rows"]:
+            ran["multirow"] += 1
+        elif st["decode_kernel_rows"]:
             ran["decode"] += 1
         elif st["prefill_kernel_rows"]:
             ran["prefill"] += 1
