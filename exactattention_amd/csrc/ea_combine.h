@@ -7,8 +7,8 @@ namespace ea {
 
 // Returns the row's stats events, the same in every lane: bit 0 the row was merged (stats[0]),
 // bit 1 it is flagged (stats[1]), bit 2 only its final rounding failed (stats[7]). The caller
-// adds them up per block.
-template <int PRE>
+// adds them up per block. MR: the multi-row kernel wrote the partials.
+template <int PRE, bool MR>
 __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
     constexpr int SLAB = 2 * PRE;  // splits per load round past PRE of them
     const int dv = P.g.head_dim_v;
@@ -77,7 +77,6 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
             *z = P.pZ[o];
         }
     };
-    const int qflag = P.mrow ? 0 : P.qinfo[row * 5 + 4];  // requested with the scalars below
     int n0, r0;
     double z0;
     load_split(0, &n0, &r0, &z0);
@@ -89,17 +88,20 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
         bad_l |= n < 0;
         if (n > 0) R_l = max(R_l, r);
     }
-    const int R = wave_max_i(R_l);
-    // a NaN/inf in q flags the row. Partials with keys carry that flag already when the multi-row
-    // kernel wrote them (no score of such a row is finite); a row without keys is looked at here
-    bool qbad = qflag != 0;
-    if (P.mrow && R == INT_MIN) {
-        const uint16_t* qr = P.q + b * P.g.q_seq_stride + (int64_t)t * P.g.q_tok_stride + (int64_t)hq * P.g.q_head_stride;
-        bool nf = false;
-        for (int i = lane; i < P.g.head_dim; i += 64) nf |= ((qr[i] >> 7) & 0xFF) == 0xFF;
-        qbad = __ballot(nf) != 0;
-    }
+    bool qbad = false;  // a NaN/inf in q flags the row
+    if constexpr (!MR) qbad = P.qinfo[row * 5 + 4] != 0;
     int flag = (__ballot(bad_l) != 0 || qbad) ? 1 : 0;
+    const int R = wave_max_i(R_l);
+    if constexpr (MR) {
+        // the multi-row kernel's partials with keys carry that flag already (no score of such a row
+        // is finite); a row without keys is looked at here
+        if (R == INT_MIN) {
+            const uint16_t* qr = P.q + b * P.g.q_seq_stride + (int64_t)t * P.g.q_tok_stride + (int64_t)hq * P.g.q_head_stride;
+            bool nf = false;
+            for (int i = lane; i < P.g.head_dim; i += 64) nf |= ((qr[i] >> 7) & 0xFF) == 0xFF;
+            if (__ballot(nf) != 0) flag = 1;
+        }
+    }
     uint16_t* o16 = (uint16_t*)P.out;
     uint32_t* o32 = (uint32_t*)P.out;
     const int64_t obase = b * P.g.o_seq_stride + (int64_t)t * P.g.o_tok_stride + (int64_t)hq * P.g.o_head_stride;
@@ -187,8 +189,9 @@ __device__ inline int combine_row(const Params& P, int64_t row, int lane) {
             else o16[obase + c] = (uint16_t)bits;
         }
     } else {
-        // per slab, both lane channels of SLAB = 16 splits requested per round: a row of 32 splits waits
-        // for 2 load latencies, of 64 for 4, and each further slab adds one for its scalars
+        // per slab of 64 splits, both lane channels of SLAB splits requested per round: a row of 32
+        // splits waits for 2 load latencies at PRE 8 and 8 at PRE 2, and each further slab adds one
+        // for its scalars
         double N[2] = {0.0, 0.0};
         float vmaxf[2] = {0.0f, 0.0f};
         if (!flag) {

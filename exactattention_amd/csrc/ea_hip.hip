@@ -583,14 +583,15 @@ __global__ void __launch_bounds__(EA_THREADS, 2) ea_split(Params P) {
 // PRE: the splits whose partials are requested in one round with their scalars. A decode step has few
 // rows of many splits, and 8 in a round; a step of many rows (prefill) has one or two pieces per
 // row and wants waves in flight instead (PRE 2: 72 registers against 157; 65,536 rows 95 -> 55 us).
-template <int PRE>
+// MR: whether the multi-row kernel wrote the partials; a branch on it cost the decode step 1 us.
+template <int PRE, bool MR>
 __global__ void __launch_bounds__(64) ea_combine(Params P) {
     // one row per 64-thread block: the merge is a chain of dependent loads, so it wants as many
     // rows in flight as the machine holds. stats[0] counts the step's rows once; the per-row
     // counters only move for flagged rows (rare), so they never serialise on one address.
     const int64_t row = blockIdx.x;
     if (row == 0 && threadIdx.x == 0 && P.stats) atomicAdd((unsigned long long*)&P.stats[0], (unsigned long long)P.rows);
-    const int ev = combine_row<PRE>(P, row, threadIdx.x);
+    const int ev = combine_row<PRE, MR>(P, row, threadIdx.x);
     if (threadIdx.x == 0 && P.stats && (ev & 2)) {
         atomicAdd((unsigned long long*)&P.stats[1], 1ull);
         if (ev & 4) atomicAdd((unsigned long long*)&P.stats[7], 1ull);
@@ -1814,8 +1815,9 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
         return rc;
     }
     if ((rc = mark(2))) return rc;
-    if (pl.rows >= 8192) hipLaunchKernelGGL(ea_combine<2>, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
-    else hipLaunchKernelGGL(ea_combine<8>, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
+    auto* const combine = pl.rows >= 8192 ? (P.mrow ? ea_combine<2, true> : ea_combine<2, false>)
+                                          : (P.mrow ? ea_combine<8, true> : ea_combine<8, false>);
+    hipLaunchKernelGGL(combine, dim3((unsigned)pl.rows), dim3(64), 0, st, P);
     rc = herr(hipGetLastError());
     if (rc) return rc;
     if ((rc = mark(3))) return rc;
