@@ -628,7 +628,7 @@ struct T2Smem {
     // per wave and channel: the N pass's partial maxima, then its 128-bit sums and lost counts
     int64_t nrw[EA_T2_WAVES][EA_MAXDV];
     uint64_t ahi[EA_T2_WAVES][EA_MAXDV], alo[EA_T2_WAVES][EA_MAXDV], aer[EA_T2_WAVES][EA_MAXDV];
-    int32_t flag;
+    int32_t flag, item;
 };
 
 __device__ void block_reduce_i128(T2Smem& S, i128* v, uint64_t* err) {
@@ -678,19 +678,27 @@ struct T2Part {
     uint64_t nhi[EA_MAXDV], nlo[EA_MAXDV], ner[EA_MAXDV];  // N_c,b in units 2^(nr_c - F), lost count
 };
 
-// The listed rows in 128-bit arithmetic, by blocks bid, bid + nb, ... Rows are split into C key
-// chunks when fewer rows are listed than there are blocks (C = blocks / rows, so one flagged row
-// takes every block instead of one): block (row slot, chunk) computes the
+// The cnt rows of a list in 128-bit arithmetic by up to EA_T2_BLOCKS blocks, each with its own slot of
+// the key scratch. Rows are split into C key chunks when fewer rows are listed than there are blocks
+// (C = blocks / rows, so one flagged row takes every block instead of one). Items (row, chunk) go
+// round by slot, or, with a counter `next`, to whichever block asks first. A block computes the
 // chunk's logits and weights and its Z and N sums, writes them as a T2Part, and the row's last
 // chunk block to finish merges the C partials. Merging moves each floored partial to the row's
 // larger base by an arithmetic right shift: floor(a 2^-s) <= a 2^-s < floor(a 2^-s) + lost, so
 // the row's sums stay of the form [acc, acc + lost count] in units of the common base, the form
-// the final rounding takes. With C = 1 the block finishes the row itself. left: only the rows that
-// the double-double pass marked (C = 1).
-__device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last, int cnt, int C, int bid, int nb, bool left) {
+// the final rounding takes. With C = 1 the block finishes the row itself. done: EA_T2_BLOCKS
+// counters, 0 at the start, of the rows' finished chunks.
+__device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last, int32_t* list, int cnt, int slot_id,
+                                        int32_t* done, int32_t* next) {
     const int tid = threadIdx.x;
+    const int C = cnt >= EA_T2_BLOCKS ? 1 : EA_T2_BLOCKS / cnt;
     const int64_t items = (int64_t)cnt * C;
-    if ((int64_t)bid >= items) return;
+    auto take = [&](int64_t mine) -> int64_t {
+        if (!next) return mine;
+        if (tid == 0) S.item = atomicAdd(next, 1);
+        __syncthreads();
+        return S.item;
+    };
     for (int i = tid; i < 256; i += EA_T2_THREADS) {
         S.T1[i] = u64_as_f64(EA_T1_BITS[i]);
         S.T2[i] = u64_as_f64(EA_T2_BITS[i]);
@@ -698,14 +706,12 @@ __device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last,
     __syncthreads();
     const int d = P.g.head_dim, dv = P.g.head_dim_v;
     const int Hq = P.g.num_q_heads, T = P.g.num_tokens;
-    int32_t* Mw = P.t2M + (int64_t)bid * P.t2_keys;
-    int64_t* Ew = P.t2E + (int64_t)bid * P.t2_keys;
+    int32_t* Mw = P.t2M + (int64_t)slot_id * P.t2_keys;
+    int64_t* Ew = P.t2E + (int64_t)slot_id * P.t2_keys;
     T2Part* parts = (T2Part*)P.t2part;
-    for (int64_t item = bid; item < items; item += nb) {
+    for (int64_t item = take(slot_id); item < items; item = take(item + EA_T2_BLOCKS)) {
         const int slot = (int)(item / C), chunk = (int)(item % C);
-        const int32_t entry = agent_load(&P.wl[slot]);
-        const int64_t row = entry & 0x7FFFFFFF;
-        if (left && entry >= 0) continue;
+        const int64_t row = agent_load(&list[slot]);
         const int64_t b = row / ((int64_t)T * Hq);
         const int t = (int)((row / Hq) % T), hq = (int)(row % Hq);
         const int hk = hq / P.grp;
@@ -1043,7 +1049,7 @@ __device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last,
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
-        if (tid == 0) s_last = atomicAdd(&P.wl_cnt[1 + slot], 1) == C - 1;
+        if (tid == 0) s_last = atomicAdd(&done[slot], 1) == C - 1;
         __syncthreads();
         if (s_last) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -1094,15 +1100,35 @@ __device__ __forceinline__ void t2_rows(const Params& P, T2Smem& S, int& s_last,
                 }
             }
             finish_row(rf);
-            if (tid == 0) P.wl_cnt[1 + slot] = 0;  // the row's count, ready for the next launch
         }
         __syncthreads();
     }
 }
 
+// Whether this block (its thread 0 asks) takes part in the 128-bit path for the rows the
+// double-double pass has left: their number, or 0, and the block's slot of the key scratch. nact blocks
+// (0 .. nact - 1) had rows of that pass, and the path starts when the last of them is done. That one
+// always takes part; the EA_T2_BLOCKS - 1 with the highest numbers wait for it. They are the last to
+// be dispatched, so that none waits in the place of one that has not started (with the first ones
+// waiting, 1024 fp32 rows took 0.89 ms instead of 0.62), and where nothing is left the launch ends
+// with its last block either way. The wait is bounded: a block that has waited 100 ms, which no pass
+// takes unless other work holds the device, goes, and leaves the rows to the others.
+__device__ __forceinline__ int t2_left(const Params& P, int nact, int* slot_id) {
+    int done = atomicAdd(&P.wl_cnt[EA_T2_DONE], 1) + 1;
+    *slot_id = min(nact - 1 - (int)blockIdx.x, EA_T2_BLOCKS - 1);
+    if (*slot_id == EA_T2_BLOCKS - 1 && done != nact) return 0;
+    const long long t0 = wall_clock64();  // 100 MHz
+    while (done < nact) {
+        if (wall_clock64() - t0 > 10000000) return 0;
+        __builtin_amdgcn_s_sleep(4);
+        done = agent_load(&P.wl_cnt[EA_T2_DONE]);
+    }
+    return agent_load(&P.wl_cnt[EA_T2_LEFT]);
+}
+
 // Tier 2: the listed rows in double-double (ea_refine.h), in EA_DD_PARTS key chunks in all when few
-// rows are listed; then, where a row stays undecided, the last block to finish takes what is left in
-// 128-bit arithmetic. Measured: the 70 rows that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
+// rows are listed; then the rows that stay undecided in 128-bit arithmetic. Measured: the 70 rows
+// that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
 // 4096-key bf16 row after a prefill step 116 -> 35 us; an empty list 4.0-4.5 us
 // in the trace; 512 blocks cost a C2 step 1.8 us, so bf16 steps, which list few rows, launch 32.
 __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
@@ -1110,25 +1136,20 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
         T2Smem t2;
         DDSmem dd;
     } S;
-    __shared__ int s_last;
+    __shared__ int s_last, s_left, s_slot;
     const int cnt = *P.wl_cnt;
     if (cnt == 0) return;  // the usual case
     // every item of a split row is in flight at once (a block each, a partial each, a count per row)
     // and no chunk is shorter than a pass of 128 keys
     const int C = cnt <= EA_T2_ROWS ? min(min(EA_DD_PARTS, (int)gridDim.x) / cnt, (P.t2_keys + EA_DD_KEYS - 1) / EA_DD_KEYS) : 1;
     dd_rows(P, S.dd, cnt, max(C, 1), (DDPart*)P.ddpart);
-    // the last of the blocks that had a row takes the rows left over: their marks in the list and their
-    // count are atomics, complete before the block's own count
-    const int64_t items = (int64_t)cnt * max(C, 1);
-    if ((int64_t)blockIdx.x >= items) return;
-    agent_done();
+    const int nact = (int)min((int64_t)cnt * max(C, 1), (int64_t)gridDim.x);
+    if ((int)blockIdx.x >= nact) return;
+    agent_done();  // the list of what is left, and the partials, whose memory the 128-bit path reuses
     __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = atomicAdd(&P.wl_cnt[EA_T2_DONE], 1) == (int)min(items, (int64_t)gridDim.x) - 1 &&
-                 agent_load(&P.wl_cnt[EA_T2_LEFT]) != 0;
+    if (threadIdx.x == 0) s_left = t2_left(P, nact, &s_slot);
     __syncthreads();
-    if (!s_last) return;
-    t2_rows(P, S.t2, s_last, cnt, 1, 0, 1, true);
+    if (s_left > 0) t2_rows(P, S.t2, s_last, P.t2left, s_left, s_slot, &P.wl_cnt[EA_T2_CHUNKS], &P.wl_cnt[EA_T2_NEXT]);
 }
 
 // force_tier2: every row straight to the 128-bit path, over EA_T2_BLOCKS blocks. A kernel of its own:
@@ -1138,8 +1159,7 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2_wide(Params P) {
     __shared__ T2Smem S;
     __shared__ int s_last;
     const int cnt = *P.wl_cnt;
-    if (cnt > 0)
-        t2_rows(P, S, s_last, cnt, cnt >= EA_T2_BLOCKS ? 1 : EA_T2_BLOCKS / cnt, (int)blockIdx.x, EA_T2_BLOCKS, false);
+    if (cnt > 0) t2_rows(P, S, s_last, P.wl, cnt, (int)blockIdx.x, &P.wl_cnt[EA_T2_CHUNKS], nullptr);
 }
 
 // Lists every row for tier 2 (ea_options.force_tier2); runs after tier 1, so nothing else appends.
@@ -1390,8 +1410,8 @@ void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsp
 // The workspace's layout for the plan's tier-1 choices, with the multi-row kernel's arrays or
 // without; returns its size. In turn: the tier-2 list and counters, tier 1's arrays, the 128-bit
 // path's, the prefill path's. When tier 2 runs, tier 1 and the prefill path are done with theirs, so
-// its double-double pass keeps its chunk partials there. They may reach into the 128-bit path's,
-// which starts after that pass.
+// its double-double pass keeps the list of the rows it leaves (Params::t2left) and its chunk partials
+// there. The partials may reach into the 128-bit path's arrays: that path starts after the pass.
 size_t lay_out(Plan* pl, const ea_geometry* g, const ea_options* o, bool mrow) {
     const int64_t R = pl->rows;
     const int dv = g->head_dim_v;
@@ -1435,7 +1455,7 @@ size_t lay_out(Plan* pl, const ea_geometry* g, const ea_options* o, bool mrow) {
         pl->off_pfscr = take((size_t)pl->nseg * pl->pf_nrb * pl->pf_nsplit * 512 * 32 * 8);
         pl->off_pfpart = take(pl->pf_nsplit > 1 ? (size_t)pl->pf_nsplit * R * (sizeof(PfPart) + 128 * 16) : 0);
     }
-    pl->off_dd = pl->off_front;
+    pl->off_dd = align_up(pl->off_front + (size_t)R * 4);  // past Params::t2left
     return pl->total = std::max(off, align_up(pl->off_dd + EA_DD_PARTS * sizeof(DDPart)));
 }
 
@@ -1679,6 +1699,7 @@ int ea_hip_attention(const ea_geometry* g, const ea_buffers* bf, const ea_option
     P.t2M = (int32_t*)(ws + pl.off_t2M);
     P.t2E = (int64_t*)(ws + pl.off_t2E);
     P.ddpart = (void*)(ws + pl.off_dd);
+    P.t2left = (int32_t*)(ws + pl.off_front);
     P.t2_keys = pl.t2_keys;
     P.pfq = (uint8_t*)(ws + pl.off_pfq);
     P.pfqm = (void*)(ws + pl.off_pfqm);

@@ -15,11 +15,14 @@ namespace ea {
 #define EA_MAXDV 128
 #define EA_T2_BLOCKS 32             // blocks of tier 2's 128-bit path
 // tier 2's counters (Params::wl_cnt): rows listed, chunks done per row (of the first EA_T2_ROWS), rows
-// the double-double pass left undecided, blocks that finished it
+// the double-double pass left undecided, blocks that finished it, items of the 128-bit path taken,
+// and that path's chunks done per row
 #define EA_T2_ROWS 192
 #define EA_T2_LEFT (1 + EA_T2_ROWS)
 #define EA_T2_DONE (2 + EA_T2_ROWS)
-#define EA_T2_CNT (3 + EA_T2_ROWS)
+#define EA_T2_NEXT (3 + EA_T2_ROWS)
+#define EA_T2_CHUNKS (4 + EA_T2_ROWS)
+#define EA_T2_CNT (EA_T2_CHUNKS + EA_T2_BLOCKS)
 #define EA_DD_BLOCKS(fp32) ((fp32) ? 512 : 32)  // of the double-double pass: two per CU where many rows are listed
 
 // ------------------------------------------------------------------------------------------------
@@ -65,6 +68,7 @@ struct Params {
     int32_t* t2M;     // EA_T2_BLOCKS * max_keys
     int64_t* t2E;     // EA_T2_BLOCKS * max_keys
     void* ddpart;     // EA_DD_PARTS chunk partials of the double-double pass (DDPart, ea_refine.h)
+    int32_t* t2left;  // rows: those that pass left undecided
     int32_t t2_keys;
     // int8-MFMA prefill path (ea_prefill.hip)
     uint8_t* pfq;     // rows * 512: q digit planes

@@ -135,8 +135,7 @@ struct DDSmem {
 
 // The listed rows, in grid-stride order; C chunks per row (C > 1 only with rows C <= EA_DD_PARTS and
 // rows C <= gridDim.x). parts: EA_DD_PARTS partials. Certified rows get their output and flag 0,
-// rows with a domain error flag 2; the rest are marked in the list and counted in
-// P.wl_cnt[EA_T2_LEFT].
+// rows with a domain error flag 2; the rest are listed in P.t2left, P.wl_cnt[EA_T2_LEFT] of them.
 __device__ inline void dd_rows(const Params& P, DDSmem& S, int cnt, int C, DDPart* parts) {
     const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int d = P.g.head_dim, dv = P.g.head_dim_v, Hq = P.g.num_q_heads, T = P.g.num_tokens;
@@ -151,7 +150,7 @@ __device__ inline void dd_rows(const Params& P, DDSmem& S, int cnt, int C, DDPar
     const int64_t items = (int64_t)cnt * C;
     for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
         const int slot = (int)(item / C), chunk = (int)(item % C);
-        const int64_t row = P.wl[slot] & 0x7FFFFFFF;
+        const int64_t row = P.wl[slot];
         const int64_t b = row / ((int64_t)T * Hq);
         const int t = (int)((row / Hq) % T), hq = (int)(row % Hq), hk = hq / P.grp;
         const int64_t tok = b * T + t;
@@ -405,8 +404,7 @@ __device__ inline void dd_rows(const Params& P, DDSmem& S, int cnt, int C, DDPar
         if (__syncthreads_or(und)) fl = 1;
         if (fl == 1) {
             if (tid == 0) {
-                atomicOr(&P.wl[slot], (int)0x80000000);  // left for the 128-bit path
-                atomicAdd(&P.wl_cnt[EA_T2_LEFT], 1);
+                agent_store(&P.t2left[atomicAdd(&P.wl_cnt[EA_T2_LEFT], 1)], (int32_t)row);
                 if (P.stats_x) atomicAdd((unsigned long long*)&P.stats_x[1], 1ull);
             }
             continue;

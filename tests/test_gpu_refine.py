@@ -86,3 +86,59 @@ def test_domain_errors_among_listed_rows(gpu):
     assert np.array_equal(flags.reshape(T, 2), exp), st
     ok = exp[None] == 0
     assert np.array_equal(got[ok], want[ok]) and not got[~ok].any(), st
+
+
+def _spread_problem(rng, B, T, Hq, Hkv, S, d):
+    """Logits of exactly +600 and -600 (alpha 1) in every row, and a few of 600.5 below the top: weights
+    1200 binades apart, which tier 1 flags and the double-double pass (800 at most) leaves."""
+    prob = _rand_problem(rng, "normal", "normal", B=B, T=T, Hq=Hq, Hkv=Hkv, S=S, d=d, dv=d)
+    prob["seq_len"][:] = S
+    prob["kv_len"][:] = np.tile(S - T + 1 + np.arange(T), B)
+    prob["q"][:] = 0
+    prob["q"][..., 0] = 0x3F80
+    t = rng.choice(np.float32([600, 599.5, -600]), size=prob["k"].shape[:3])
+    t[:, :, :2] = [600, -600]
+    prob["k"][:] = 0
+    hi = np.float32(np.round(t / 8) * 8)  # bf16 keeps 8 bits: t as two terms
+    prob["k"][..., 0] = hi.view(np.uint32) >> 16
+    prob["q"][..., 1] = 0x3F80
+    prob["k"][..., 1] = np.float32(t - hi).view(np.uint32) >> 16
+    return prob
+
+
+@pytest.mark.parametrize("out", ["bf16", "fp32"])
+@pytest.mark.parametrize("B,T,Hq,Hkv,S,d", [(1, 1, 3, 1, 5000, 64), (1, 1, 4, 1, 90, 128), (2, 5, 8, 2, 700, 64),
+                                            (3, 1, 64, 4, 300, 128), (8, 1, 40, 8, 200, 64)])
+def test_rows_left_to_the_128_bit_path(gpu, B, T, Hq, Hkv, S, d, out):
+    """Every row past the double-double pass: few rows (their keys split into chunks), more than there
+    are blocks, and more than that pass counts chunks for; the 128-bit path certifies them all."""
+    rng = np.random.default_rng(S)
+    prob = _spread_problem(rng, B, T, Hq, Hkv, S, d)
+    ab = int(np.float32(1).view(np.uint32))
+    want, wflags = _oracle(prob, ab, out)
+    got, flags, st = _run(prob, ab, out)
+    assert st["tier2_wide_rows"] == flags.size == st["tier1_flagged"] == st["tier2_certified"], st
+    assert not flags.any() and not np.any(wflags)
+    assert np.array_equal(got, want), st
+
+
+def test_rows_left_are_shared_by_the_blocks(gpu):
+    """64 rows past the double-double pass take little longer than on force_tier2's 32 blocks (a single block
+    took 32 times as long), and so does one long row, whose keys are split."""
+    import torch
+    from exactattention_amd.hip import DeviceProblem, launch_hip
+    rng = np.random.default_rng(1)
+    ab = int(np.float32(1).view(np.uint32))
+    for B, Hq, S in ((8, 8, 2000), (1, 1, 30000)):
+        dp = DeviceProblem(_spread_problem(rng, B, 1, Hq, 1, S, 64))
+        ms = {}
+        for force in (False, True):
+            for _ in range(3):
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                launch_hip(dp, ab, force_tier2=force)
+                b.record()
+                torch.cuda.synchronize()
+                ms[force] = min(ms.get(force, 1e9), a.elapsed_time(b))
+        assert not dp.flags.any()
+        assert ms[False] < 4 * ms[True], (B, S, ms)
