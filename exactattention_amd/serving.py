@@ -23,6 +23,7 @@ Every call enqueues on torch's current stream and copies its result to the host 
 from __future__ import annotations
 
 import ctypes
+import operator
 
 import numpy as np
 
@@ -326,19 +327,32 @@ class PagedKVCache:
                    "ea_hip_kv_digits_update")
 
 
-def _equal_runs(ql):
+def _equal_runs(ql, heads=None, head_dim=128, longest=0):
     """The batch's runs of consecutive sequences with equal token counts, as (first, past the last)
     pairs, where one launch per run beats one padded to the longest chunk, else None. A single run
     needs no padding at all (4 x 5 tokens on 1000-key prefixes 197 -> 158 us a call, 300 tokens on
     4000 keys 650 -> 625). Two or three pay for their extra launches when padding would more than
-    double the rows, to 512 or more: decode tokens padded to a prompt chunk's length run its
+    double the tokens, to 512 or more: decode tokens padded to a prompt chunk's length run its
     long serial blocks (150 tokens beside 11 decode tokens on 4000-key prefixes 937 -> 545 us, 64
-    beside 8 on 2000 399 -> 380); at 4 x 64 rows the two come out even (290, 302)."""
-    runs = [0] + [i for i in range(1, len(ql)) if ql[i] != ql[i - 1]] + [len(ql)]
-    n = len(runs) - 1
-    if n == 1 or (n <= 3 and len(ql) * max(ql) > 2 * sum(ql) and len(ql) * max(ql) >= 512):
-        return list(zip(runs[:-1], runs[1:]))
-    return None
+    beside 8 on 2000 399 -> 380); at 4 x 64 tokens the two come out even (290, 302). The launches of
+    three runs cost the host about 20 us more than padding. With 128-dim heads, whose padded batch runs
+    on the int8 kernel, `heads` query heads and prefixes of up to `longest` keys decide (us a call among
+    others, padded -> three runs): 64 tokens between 5 and 5 decode tokens, 16 heads, 300 keys 236 ->
+    257, 3000 keys 243 -> 264 (but alone 413 -> 359), 5000 keys 0.83 times, 9000 keys 0.60; 4 heads
+    9000 keys 287 -> 310; 100 tokens between 12 and 12, 32 heads, 300 keys 259 -> 275, 1000 keys 0.90
+    times, 2000 keys 0.64; 64 heads, 300 keys 0.96, 1000 keys 0.69."""
+    n = 1 + sum(map(operator.ne, ql, ql[1:]))
+    if n == 1:
+        return [(0, len(ql))]
+    tokens = len(ql) * max(ql)
+    if n > 3 or tokens < 512 or tokens <= 2 * sum(ql):
+        return None
+    if n == 3 and heads is not None and head_dim == 128:
+        rows = tokens * heads
+        if not (rows >= 8192 and longest >= 3000 or rows >= 65536 and longest >= 1000 or rows >= 131072):
+            return None
+    cut = [0] + [i for i in range(1, len(ql)) if ql[i] != ql[i - 1]] + [len(ql)]
+    return list(zip(cut[:-1], cut[1:]))
 
 
 class ExactAttentionBackend:
@@ -474,15 +488,16 @@ class ExactAttentionBackend:
         plan = c._plan_append(seqs, ql, key, value, checked=True)
         lens = np.asarray([c.length[s] for s in seqs], dtype=np.int32)
         mine = [lens, np.asarray(seqs, dtype=np.int64) * c.max_pages, np.asarray(seqs, dtype=np.int32)]
-        plain = query.dim() == 3 and query.element_size() == 2 and query.device == c.k.device
-        runs = _equal_runs(ql) if T > 1 and plain else None
+        runs = None
         if T > 1:
+            if query.dim() == 3 and query.element_size() == 2 and query.device == c.k.device:
+                runs = _equal_runs(ql, Hq, d, max(prefix))
             start = np.concatenate([[0], np.cumsum(ql)])
             b_of = np.repeat(np.arange(B), ql)
             j_of = np.arange(ntok) - start[b_of]
-            seen = (np.asarray(prefix)[b_of] + j_of + 1).astype(np.int32)
+            seen = np.asarray(prefix, dtype=np.int32)[b_of] + j_of + 1
             if runs is not None:
-                mine.append(seen)
+                mine.append(seen.astype(np.int32))
             else:
                 kvl_h = np.zeros(B * T, dtype=np.int32)
                 kvl_h[b_of * T + j_of] = seen

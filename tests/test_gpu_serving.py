@@ -466,13 +466,16 @@ def test_kv_append_scatter(gpu, row_elems):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d,out", [(128, "bf16"), (64, "fp32")])
-def test_forward_runs_match_oracle(gpu, d, out):
+def test_forward_runs_match_oracle(gpu, monkeypatch, d, out):
     """forward() on batches whose runs of equal token counts are launched one by one: one run, a
     chunk after and between decode tokens (the outer runs share one shape but not their lengths),
     and a batch that stays padded; query views off 16-byte alignment. Then the exact tier on every
     row of every run, after the caller has overwritten its query, gives the same bits."""
     import torch
+    from exactattention_amd import serving
     from exactattention_amd.serving import ExactAttentionBackend, PagedKVCache, _equal_runs
+    # three runs also at sizes where 128-dim heads are padded
+    monkeypatch.setattr(serving, "_equal_runs", lambda ql, *sizes: _equal_runs(ql))
     rng = np.random.default_rng(91)
     Hq, Hkv = 4, 2
     ab = default_alpha_bits(d)

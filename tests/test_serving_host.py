@@ -232,3 +232,22 @@ def test_check_flags_never_passes_flag_one():
         be.check_flags(torch.tensor([[0, 1], [0, 0]], dtype=torch.uint8))
     with pytest.raises(ExactAttentionDomainError):
         be.check_flags(torch.tensor([[0, 2]], dtype=torch.uint8))
+
+
+def test_equal_runs_of_a_batch():
+    """Which batches forward() launches run by run: one run always, two where padding would more than
+    double 512 tokens or more, three with 128-dim heads only where the padded kernel's work is large."""
+    from exactattention_amd.serving import _equal_runs
+    assert _equal_runs([5, 5, 5], 16, 128, 10) == [(0, 3)]
+    assert _equal_runs([1] * 11 + [150], 16, 128, 300) == [(0, 11), (11, 12)]
+    assert _equal_runs([64, 1, 1], 16, 128, 300) is None                     # 192 padded tokens
+    assert _equal_runs([300, 250, 250], 16, 128, 300) is None                # padding adds little
+    mid = [1] * 5 + [64] + [1] * 5
+    three = [(0, 5), (5, 6), (6, 11)]
+    assert _equal_runs(mid) == _equal_runs(mid, 16, 64, 300) == _equal_runs(mid, 16, 128, 3000) == three
+    assert _equal_runs(mid, 16, 128, 2999) is None
+    assert _equal_runs(mid, 8, 128, 9000) is None                            # 5632 padded rows
+    wide = [1] * 12 + [100] + [1] * 12
+    assert _equal_runs(wide, 32, 128, 1000) and _equal_runs(wide, 64, 128, 0)
+    assert _equal_runs(wide, 32, 128, 999) is None
+    assert _equal_runs([1, 64, 1, 64] * 3, 64, 128, 9000) is None            # many runs
