@@ -1391,20 +1391,27 @@ void choose_splits(int64_t items, int maxlen, int splits, int* nsplit, int* spli
 // on 4 KV heads 114, 73, 55.5, 65). Steps that fill the device take splits
 // of at most 512 keys, so that the equal-share plan (taken past one round of resident blocks) can
 // even out sequences of different lengths in shares of 8 tiles, while the partials stay below
-// MROW_PART.
-void choose_splits_mrow(const Plan& pl, int maxlen, int dv, int splits, int* nsplit, int* split_len) {
+// MROW_PART. But that plan costs a launch and a prologue per piece, about 8 us (4 tiles of 4 rows, one
+// of 16), so short splits are kept to one round where that gives a block no more tiles than that above
+// its share, and at most 10 (16/8 or 8/8 heads, one token, plan -> one round: 32 x 300 keys 42.3 ->
+// 31.0 us, 32 x 700 50.0 -> 41.2, 64 x 300 46.5 -> 40.6, ragged to 900 keys 49.6 -> 38.6; but 24 rows, 20
+// x 400 keys 100 -> 112).
+void choose_splits_mrow(const Plan& pl, Tier1& mr, int maxlen, int dv, int splits) {
     int ns = splits;
     if (ns == 0) {
         const int64_t MROW_PART = 32 << 20;
-        const int64_t units = (int64_t)pl.nseg * pl.mr.nrb;
+        const int64_t units = (int64_t)pl.nseg * mr.nrb;
         const int64_t items = pl.r_seg <= 8 ? (int64_t)pl.nseg * ((pl.r_seg + 1) / 2) : 2 * units;
         const int64_t tiles = ((int64_t)maxlen + EA_TILE - 1) / EA_TILE;
         ns = 1;
         while (items * ns < 1024 && (int64_t)maxlen / (ns * 2) >= 64 && (int64_t)ns * ns <= 2 * tiles) ns *= 2;
         while (items * ns >= 1024 && (int64_t)maxlen / ns > 512 && 2 * ns * pl.rows * dv * 8 <= MROW_PART) ns *= 2;
         while ((int64_t)maxlen / ns > 2048 && ns < 1024) ns *= 2;
+        const int64_t ROUND = 512, fit = ROUND / std::max<int64_t>(units, 1);  // 2 resident blocks per CU
+        const int64_t chain = fit > 0 ? (tiles + fit - 1) / fit : tiles, share = (units * tiles + ROUND - 1) / ROUND;
+        if (ns > fit && fit > 0 && chain <= 10 && chain - share <= 16 / mr.rb) ns = (int)fit;
     }
-    split_tiles(maxlen, ns, nsplit, split_len);
+    split_tiles(maxlen, ns, &mr.nsplit, &mr.split_len);
 }
 
 // The workspace's layout for the plan's tier-1 choices, with the multi-row kernel's arrays or
@@ -1525,7 +1532,20 @@ int make_plan(const ea_geometry* g, const ea_options* o, Plan* pl) {
     const size_t without = lay_out(pl, g, o, false);
     if (!pl->mrow) return 0;
     mr.nrb = (pl->r_seg + mr.rb - 1) / mr.rb;
-    choose_splits_mrow(*pl, maxlen, g->head_dim_v, o->splits, &mr.nsplit, &mr.split_len);
+    choose_splits_mrow(*pl, mr, maxlen, g->head_dim_v, o->splits);
+    // Row blocks of half the rows while their grid is at most a block per CU: a wave's chain of steps
+    // is what such a step waits for, and it is shorter with fewer rows. 16 rows, 16 -> 4 a block: 8
+    // segments of 100 keys 32.7 -> 25.8 us a step (29.5 on ea_decode), of 1000 33.2 -> 27.0; one of 16K 58.7
+    // -> 41.0 (56.4); 8 rows, 8 -> 4: 8 segments of 2000 keys 30.2 -> 28.3. Past it they only read K and V
+    // more often: 8 segments of 16K keys 63 -> 74.
+    while (mr.rb > 4) {
+        Tier1 half = mr;
+        half.rb = mr.rb / 2;
+        half.nrb = (pl->r_seg + half.rb - 1) / half.rb;
+        choose_splits_mrow(*pl, half, maxlen, g->head_dim_v, o->splits);
+        if ((int64_t)pl->nseg * half.nrb * half.nsplit > 256) break;
+        mr = half;
+    }
     mr.dq = dq_fits(mr.nrb);
     // A step that fits the allocation-free entry point's array with the other kernel's arrays fits it
     // with this one's too: with fewer splits where the caller left them open, or without the
@@ -1636,7 +1656,7 @@ int ea_hip_workspace_size(const ea_geometry* g, const ea_options* o, size_t* byt
 }
 
 int ea_hip_step_route(const ea_geometry* g, const ea_buffers* bf, const ea_options* o, int32_t* kernel,
-                      int32_t* nsplit, int32_t* ordered) {
+                      int32_t* nsplit, int32_t* ordered, int32_t* block_rows) {
     Plan pl;
     int rc = make_plan(g, o, &pl);
     if (rc) return rc;
@@ -1652,6 +1672,7 @@ int ea_hip_step_route(const ea_geometry* g, const ea_buffers* bf, const ea_optio
     if (kernel) *kernel = k;
     if (nsplit) *nsplit = pl.prefill ? pl.pf_nsplit : P.nsplit;
     if (ordered) *ordered = !pl.prefill && usable_merge_order(P, pl, o) != nullptr;
+    if (block_rows) *block_rows = P.rb;
     return 0;
 }
 

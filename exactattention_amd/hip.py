@@ -79,7 +79,7 @@ def load():
         lib.ea_hip_reads_kv_digits.restype = ctypes.c_int
         lib.ea_hip_step_route.argtypes = [ctypes.POINTER(Geometry), ctypes.POINTER(Buffers), ctypes.POINTER(Options),
                                           ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32),
-                                          ctypes.POINTER(ctypes.c_int32)]
+                                          ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
         lib.ea_hip_step_route.restype = ctypes.c_int
         lib.ea_hip_attention.argtypes = [ctypes.POINTER(Geometry), ctypes.POINTER(Buffers), ctypes.POINTER(Options),
                                          P, ctypes.c_size_t, P]
@@ -149,14 +149,15 @@ def workspace_size(g: dict, splits: int = 0, out_fp32: bool = False, kernel: int
 ROUTES = {1: "prefill", 2: "decode", 3: "general", 4: "multirow"}
 
 
-def step_route(g: dict, ptrs: dict, **opt) -> tuple[str, int, bool]:
-    """The tier-1 kernel a step on these pointers takes, its KV splits, and whether a merge order in
-    `opt` (ea_options fields) is followed (ea_hip_step_route; nothing runs on the device)."""
-    out = [ctypes.c_int32(-1) for _ in range(3)]
+def step_route(g: dict, ptrs: dict, **opt) -> tuple[str, int, bool, int]:
+    """The tier-1 kernel a step on these pointers takes, its KV splits, whether a merge order in
+    `opt` (ea_options fields) is followed, and its rows per block (ea_hip_step_route; nothing runs
+    on the device)."""
+    out = [ctypes.c_int32(-1) for _ in range(4)]
     _check(load().ea_hip_step_route(ctypes.byref(geometry(g)), ctypes.byref(Buffers(**ptrs)),
                                     ctypes.byref(Options(tier2=1, **opt)), *(ctypes.byref(x) for x in out)),
            "ea_hip_step_route")
-    return ROUTES[out[0].value], out[1].value, bool(out[2].value)
+    return ROUTES[out[0].value], out[1].value, bool(out[2].value), out[3].value
 
 
 class DeviceProblem:

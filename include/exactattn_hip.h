@@ -165,11 +165,12 @@ int ea_hip_reads_kv_digits(const ea_geometry* g, const ea_options* o, int32_t* r
  * (host logic only: pointers are looked at for their alignment, nothing is read): *kernel =
  * EA_KERNEL_PREFILL, EA_KERNEL_DECODE (the d = 128 decode kernel), EA_KERNEL_GENERAL or
  * EA_ROUTE_MULTIROW; *nsplit the KV splits that kernel takes (an equal-share plan, decided by the
- * device's size, replaces them); *ordered = 1 when o->merge_order is followed on those splits. Each output may be NULL. Returns 0 or the
+ * device's size, replaces them); *ordered = 1 when o->merge_order is followed on those splits; *block_rows the
+ * rows of a block (the multi-row kernel's 4, 8 or 16; 0 for the prefill kernel). Each output may be NULL. Returns 0 or the
  * negative codes of ea_hip_workspace_size, -1 for NULL buffers. No reference counterpart. */
 #define EA_ROUTE_MULTIROW 4
 int ea_hip_step_route(const ea_geometry* g, const ea_buffers* b, const ea_options* o, int32_t* kernel,
-                      int32_t* nsplit, int32_t* ordered);
+                      int32_t* nsplit, int32_t* ordered, int32_t* block_rows);
 
 /* Enqueue one certified attention step on `stream`: q prep (inside the tier-1 kernel on the d =
  * 128 decode kernel's uniform grid), tier-1 split kernel, combine with

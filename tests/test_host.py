@@ -448,7 +448,7 @@ def test_merge_order_is_read_only_at_its_own_length(d):
                 ptrs[n] += change.get(n, 0)
             for splits in (0, 3, 40, 100):
                 rc, _, reported = _ws(g, splits)
-                kernel, ns, ordered = hip.step_route(g, ptrs, splits=splits, merge_order=1 << 20)
+                kernel, ns, ordered, _ = hip.step_route(g, ptrs, splits=splits, merge_order=1 << 20)
                 assert rc == 0 and (not ordered or (ns == reported and ns <= 64)), (change, S, splits, kernel, ns)
                 assert ordered or ns != reported or ns > 64, (change, S, splits, kernel, ns)
                 assert not hip.step_route(g, ptrs, splits=splits)[2]
@@ -492,3 +492,19 @@ def test_multi_row_steps_fit_where_the_general_kernel_fits():
         assert nb <= NOALLOC_BYTES or want > NOALLOC_BYTES, (B, T, Hkv, grp, d, dv, S, splits, nb, want)
         near += NOALLOC_BYTES * 3 // 4 < want <= NOALLOC_BYTES
     assert near > 50, near
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,d,S,ns,rb", [
+    # short steps of many units stay within one round of 512 blocks instead of the equal-share plan
+    (32, 1, 8, 8, 128, 300, 2, 4), (64, 1, 8, 8, 128, 300, 1, 4), (20, 1, 8, 8, 128, 700, 3, 4),
+    (32, 1, 16, 8, 128, 900, 2, 4), (48, 1, 4, 4, 128, 700, 2, 4), (128, 1, 8, 8, 64, 300, 1, 4),
+    # unless a block would take much more than its share, or more than 10 tiles
+    (20, 12, 16, 8, 128, 400, 2, 16), (32, 1, 64, 8, 128, 4096, 8, 8), (24, 1, 8, 4, 128, 2600, 5, 4),
+    # 16-row blocks only where halving them makes more than 256 blocks, as down to 8 and 4
+    (1, 1, 128, 8, 128, 100, 1, 4), (1, 1, 16, 1, 128, 16384, 32, 4), (1, 1, 128, 8, 128, 16384, 32, 16),
+    (1, 1, 64, 8, 128, 2000, 16, 4), (1, 1, 64, 8, 128, 30000, 59, 8), (70, 1, 32, 2, 64, 64, 1, 16),
+    (70, 1, 16, 2, 64, 64, 1, 8), (8, 8, 16, 8, 128, 16384, 32, 16)])
+def test_multi_row_blocks_and_splits(B, T, Hq, Hkv, d, S, ns, rb):
+    from exactattention_amd import hip
+    g, ptrs = _step_geom(B, T, Hq, Hkv, d, S)
+    assert hip.step_route(g, ptrs) == ("multirow", ns, False, rb)
