@@ -26,6 +26,9 @@ def test_many_listed_rows(gpu, T, S, kind):
     assert st["tier2_certified"] == st["tier1_flagged"], st
     if kind == "normal":
         assert st["tier1_flagged"] > 32, st
+    # decided by the double-double pass itself, but for terms a window apart (wide) or past 2^-120 (outlier)
+    assert st["tier2_wide_rows"] == 0 or kind in ("wide", "outlier"), st
+    assert kind != "wide" or st["tier2_wide_rows"] > 0, st
 
 
 @pytest.mark.parametrize("d,dv", [(128, 128), (64, 64), (40, 6)])
@@ -60,7 +63,7 @@ def test_few_listed_rows(gpu, d, dv, S):
         got, flags, st = _run(prob, ab, out)
         assert not np.any(wflags) and not flags.any(), st
         assert np.array_equal(got, want), st
-        assert st["tier2_certified"] == st["tier1_flagged"], st
+        assert st["tier2_certified"] == st["tier1_flagged"] == 1 and st["tier2_wide_rows"] == 0, st
 
 
 def test_domain_errors_among_listed_rows(gpu):
