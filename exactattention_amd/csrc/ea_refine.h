@@ -88,9 +88,12 @@ __device__ inline bool dd_quotient(const DD& n, const DD& z, double adds, int fp
     const double d0 = two_sum(nh, -p1, &e0);
     const double rest = ((nl - m * z.lo) - e1) + e0;
     const double r = d0 + rest;
-    const double err = (fabs(d0) + fabs(rest) + fabs(nl) + fabs(m * z.lo) + fabs(e1) + fabs(e0)) * 0x1p-50 + en + m * ez;
+    // the last term covers products here, and parts of the sums scaled down with a row's reference,
+    // that fall below the smallest numbers (2^-1074 each)
+    const double err = (fabs(d0) + fabs(rest) + fabs(nl) + fabs(m * z.lo) + fabs(e1) + fabs(e0)) * 0x1p-50 + en + m * ez + 0x1p-1000;
+    const bool exact = nl == 0.0 && n.mag == 0.0 && n.err == 0.0 && z.lo == 0.0 && z.mag == 0.0 && z.err == 0.0;
     uint64_t k = mb >> S;  // the format's value below the midpoint
-    if (err == 0.0 && r == 0.0) k += k & 1;  // an exact tie: to even
+    if (exact && d0 == 0.0 && e0 == 0.0 && e1 == 0.0) k += k & 1;  // a tie: to even
     else if (r > err) ++k;
     else if (!(r < -err)) return false;
     const uint32_t mag = (uint32_t)(k - ((uint64_t)(1023 - 127) << (52 - S)));

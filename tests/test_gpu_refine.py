@@ -145,3 +145,29 @@ def test_rows_left_are_shared_by_the_blocks(gpu):
                 ms[force] = min(ms.get(force, 1e9), a.elapsed_time(b))
         assert not dp.flags.any()
         assert ms[False] < 4 * ms[True], (B, S, ms)
+
+
+def test_reference_moves_past_the_number_range(gpu):
+    """A row's reference exponent moves by 790 binades twice, each move in another pass of 128 keys (more
+    rows than are split into chunks): the first pass's terms end below the smallest fp64 number. Channel
+    0's quotient is an exact tie; in channels 1 and 2 those terms put it below and above, by 2^-1580."""
+    from exactattention_amd.hip import attention_problem
+    rng = np.random.default_rng(0)
+    prob = _rand_problem(rng, "normal", "normal", B=10, T=1, Hq=4, Hkv=2, S=384, d=64, dv=64)
+    prob["seq_len"][:] = prob["kv_len"][:] = 384
+    prob["q"][:] = 0
+    prob["q"][..., :2] = 0x3F80
+    prob["k"][:] = 0
+    for p, (hi, lo) in enumerate(((0, 0), (784, 6), (1576, 4))):
+        keys = slice(128 * p, 128 * p + 128)
+        prob["k"][:, :, keys, 0] = int(np.float32(hi).view(np.uint32)) >> 16
+        prob["k"][:, :, keys, 1] = int(np.float32(lo).view(np.uint32)) >> 16
+        prob["v"][:, :, keys, :3] = (0x3F80 + np.arange(128) % 2)[:, None]  # 1 and 1 + 2^-7: the mean is a tie
+    prob["v"][:, :, :128, 1] = 0x3F80
+    prob["v"][:, :, :128, 2] = 0x3F81
+    ab = int(np.float32(1).view(np.uint32))
+    want, _ = _oracle(prob, ab)
+    got, flags, st = attention_problem(prob, alpha_bits=ab)
+    assert st["tier1_flagged"] == flags.size, st
+    assert not flags.any() and np.array_equal(got, want), st
+    assert (got[..., :3] == [0x3F80, 0x3F80, 0x3F81]).all()
