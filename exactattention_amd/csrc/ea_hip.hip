@@ -1259,6 +1259,25 @@ __global__ void __launch_bounds__(64) ea_kat_wave_max(int64_t nwaves, const int3
     out[blockIdx.x * 64 + threadIdx.x] = v;
 }
 
+// One wave per case, lane l = 16 x + c: A and B operands a[64 w + l], b[64 w + l], accumulators
+// c[256 w + 64 i + l]. o16: v_mfma_f64_16x16x4, D register i in lane order; o4: v_mfma_f64_4x4x4 on
+// accumulator 0.
+__global__ void __launch_bounds__(64) ea_kat_mfma_f64(int64_t n, const double* a, const double* b, const double* c,
+                                                      double* o16, double* o4) {
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    const int64_t w = blockIdx.x;
+    if (w >= n) return;
+    const int l = threadIdx.x;
+    v4d acc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = c[256 * w + 64 * i + l];
+    const double x = a[64 * w + l], y = b[64 * w + l];
+    o4[64 * w + l] = __builtin_amdgcn_mfma_f64_4x4x4f64(x, y, acc[0], 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o16[256 * w + 64 * i + l] = acc[i];
+}
+
 __global__ void ea_kat_round(int64_t n, const double* x, const double* r, int32_t fp32, uint32_t* bits, int32_t* ok) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -2066,6 +2085,14 @@ int ea_hip_kat_weight(int64_t n, const uint32_t* t_bits, int32_t* M, int64_t* E,
 int ea_hip_kat_wave_max(int64_t nwaves, const int32_t* in, int32_t* out, ea_stream_t stream) {
     if (nwaves <= 0) return nwaves < 0 ? -1 : 0;
     hipLaunchKernelGGL(ea_kat_wave_max, dim3((unsigned)nwaves), dim3(64), 0, (hipStream_t)stream, nwaves, in, out);
+    return herr(hipGetLastError());
+}
+
+int ea_hip_kat_mfma_f64(int64_t n, const double* a, const double* b, const double* c, double* o16, double* o4,
+                        ea_stream_t stream) {
+    if (n <= 0) return n < 0 ? -1 : 0;
+    if (n > (1 << 24) || !a || !b || !c || !o16 || !o4) return -1;
+    hipLaunchKernelGGL(ea_kat_mfma_f64, dim3((unsigned)n), dim3(64), 0, (hipStream_t)stream, n, a, b, c, o16, o4);
     return herr(hipGetLastError());
 }
 

@@ -119,6 +119,8 @@ def load():
         lib.ea_hip_kat_rn32_prod.restype = ctypes.c_int
         lib.ea_hip_kat_wave_max.argtypes = [ctypes.c_int64, P, P, P]
         lib.ea_hip_kat_wave_max.restype = ctypes.c_int
+        lib.ea_hip_kat_mfma_f64.argtypes = [ctypes.c_int64] + [P] * 5 + [P]
+        lib.ea_hip_kat_mfma_f64.restype = ctypes.c_int
         lib.ea_hip_version.restype = ctypes.c_char_p
         _lib = lib
     return _lib

@@ -276,6 +276,14 @@ int ea_hip_kat_round(int64_t n, const double* x, const double* r, int32_t fp32, 
  * (the DPP reduction the split kernel uses for row maxima and flags). No reference counterpart:
  * the reference's reductions are Triton's tl.max. */
 int ea_hip_kat_wave_max(int64_t nwaves, const int32_t* in, int32_t* out, ea_stream_t stream);
+/* ea_hip_kat_mfma_f64: the two fp64 matrix instructions the multi-row kernel's error bounds rest on,
+ * one case per wave. Lane l = 16 x + c gives a[64 w + l], b[64 w + l] and the accumulators
+ * c[256 w + 64 i + l]. 16x16x4 (o16, 256 a case): A row c, K x; B K x, column c; register i of lane l
+ * is row 4 i + x, column c. 4x4x4 (o4, 64 a case, accumulator 0): within each block c / 4, A row c % 4,
+ * K x; B K x, column c % 4; lane l is row x, column c % 4. Each element is the chain of four fma()
+ * over ascending K. n <= 2^24. No reference counterpart. */
+int ea_hip_kat_mfma_f64(int64_t n, const double* a, const double* b, const double* c, double* o16, double* o4,
+                        ea_stream_t stream);
 int ea_hip_kat_round_ratio(int64_t n, const uint64_t* a_hi, const uint64_t* a_lo, const uint64_t* b_hi,
                            const uint64_t* b_lo, const int32_t* E, const int32_t* neg, int32_t fp32, uint32_t* bits,
                            int32_t* overflow, ea_stream_t stream);

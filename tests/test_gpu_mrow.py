@@ -2,6 +2,8 @@
 (16 keys per wave, 64 per tile), splits and head sizes, against the oracle. Every result is
 certified, so the bar is equal bits."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -167,3 +169,55 @@ def test_combine_of_many_rows(gpu, splits):
     for B, S in ((3, 500), (128, 128), (127, 128)):
         prob = _rand_problem(rng, "normal", "outlier", B=B, T=1, Hq=32, Hkv=16, S=S, d=128, dv=128)
         _check(prob, default_alpha_bits(128), splits=splits, mrow=B != 128)  # 128 x 16 x 2 tiles: ea_decode's
+
+
+def _fma():
+    f = ctypes.CDLL("libm.so.6").fma
+    f.argtypes, f.restype = [ctypes.c_double] * 3, ctypes.c_double
+    return f
+
+
+@pytest.mark.parametrize("kind", ["normal", "wide", "cancel", "subnormal"])
+def test_matrix_instructions_are_fma_chains(gpu, kind):
+    """v_mfma_f64_16x16x4 and 4x4x4 give, bit for bit, chains of four single-rounding FMAs in ascending
+    K order, on which the kernel's error bounds rest: random operands, exponents far apart, sums that
+    cancel to their last bits, and operands and sums that are subnormal."""
+    import torch
+    from exactattention_amd import hip
+    rng = np.random.default_rng(12)
+    n = 24
+    a, b, c = rng.standard_normal((n, 64)), rng.standard_normal((n, 64)), rng.standard_normal((n, 4, 64))
+    if kind == "wide":
+        a, b = np.ldexp(a, rng.integers(-300, 300, a.shape)), np.ldexp(b, rng.integers(-300, 300, b.shape))
+        c = np.ldexp(c, rng.integers(-500, 500, c.shape))
+    elif kind == "cancel":
+        # K pairs (0, 1) and (2, 3) of nearly opposite products, and an accumulator near minus the rest
+        a[:, 16:32], b[:, 16:32] = -a[:, :16], b[:, :16] * (1 + rng.integers(-4, 5, (n, 16)) * 2.0 ** -52)
+        a[:, 48:], b[:, 48:] = -a[:, 32:48], b[:, 32:48] * (1 + rng.integers(-4, 5, (n, 16)) * 2.0 ** -52)
+        c *= 2.0 ** -50
+    elif kind == "subnormal":
+        a, b = np.ldexp(a, rng.integers(-560, -500, a.shape)), np.ldexp(b, rng.integers(-560, -500, b.shape))
+        c = np.ldexp(c, rng.integers(-1080, -1030, c.shape))
+    lib = hip.load()
+    dev = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (a, b, c)]
+    o16 = torch.zeros((n, 4, 64), dtype=torch.float64, device="cuda")
+    o4 = torch.zeros((n, 64), dtype=torch.float64, device="cuda")
+    assert lib.ea_hip_kat_mfma_f64(n, *(t.data_ptr() for t in dev), o16.data_ptr(), o4.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    fma = _fma()
+    w16, w4 = np.zeros((n, 4, 64)), np.zeros((n, 64))
+    for w in range(n):
+        A, B = a[w].reshape(4, 16), b[w].reshape(4, 16)  # [K][row or column]
+        for x in range(4):
+            for col in range(16):
+                for i in range(4):
+                    s = c[w, i, 16 * x + col]
+                    for k in range(4):
+                        s = fma(A[k, 4 * i + x], B[k, col], s)
+                    w16[w, i, 16 * x + col] = s
+                s = c[w, 0, 16 * x + col]
+                for k in range(4):
+                    s = fma(A[k, col // 4 * 4 + x], B[k, col], s)
+                w4[w, 16 * x + col] = s
+    assert np.array_equal(o16.cpu().numpy().view(np.uint64), w16.view(np.uint64))
+    assert np.array_equal(o4.cpu().numpy().view(np.uint64), w4.view(np.uint64))
