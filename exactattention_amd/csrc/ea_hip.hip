@@ -10,8 +10,8 @@
 //                rigorous error bounds. Writes one partial per (split, row).
 //   ea_combine   merges the split partials in the caller's order and certifies RN(N/Z) per
 //                channel; appends rows it cannot certify to the tier-2 work list
-//   ea_tier2     per listed row: a double-double pass with error bounds; for the rows it leaves,
-//                128-bit windowed scores, 128-bit exp2 enclosure, 128-bit fixed-point Z and N with
+//   ea_tier2     per listed row: a double-double pass with error bounds; for the rows it leaves, in the
+//                same launch, 128-bit windowed scores, 128-bit exp2 enclosure, 128-bit fixed-point Z and N with
 //                counted truncation, exact final rounding
 // Reference behaviour: src/exactattn/triton_kernels.py:1324-1519 (split, combine, tier 2,
 // host fallback) and docs/SPEC.md (the definition the bits must equal).
@@ -582,7 +582,8 @@ __global__ void __launch_bounds__(EA_THREADS, 2) ea_split(Params P) {
 // ------------------------------------------------------------------------------------------------
 // PRE: the splits whose partials are requested in one round with their scalars. A decode step has few
 // rows of many splits, and 8 in a round; a step of many rows (prefill) has one or two pieces per
-// row and wants waves in flight instead (PRE 2: 72 registers against 157; 65,536 rows 95 -> 55 us).
+// row and wants waves in flight instead (PRE 2: 72 registers against 157; 65,536 rows of 64-dim heads,
+// two pieces each, 92 -> 53 us).
 // MR: whether the multi-row kernel wrote the partials; a branch on it cost the decode step 1 us.
 template <int PRE, bool MR>
 __global__ void __launch_bounds__(64) ea_combine(Params P) {
@@ -1128,9 +1129,10 @@ __device__ __forceinline__ int t2_left(const Params& P, int nact, int* slot_id) 
 
 // Tier 2: the listed rows in double-double (ea_refine.h), in EA_DD_PARTS key chunks in all when few
 // rows are listed; then the rows that stay undecided in 128-bit arithmetic. Measured: the 70 rows
-// that a 2048-row causal head in fp32 leaves, 900 -> 72 us; one
-// 4096-key bf16 row after a prefill step 116 -> 35 us; an empty list 4.0-4.5 us
-// in the trace; 512 blocks cost a C2 step 1.8 us, so bf16 steps, which list few rows, launch 32.
+// that a 2048-row causal head in fp32 leaves, 840 -> 66 us; one
+// 4096-key bf16 row after a prefill step 116 -> 35 us; an empty list 4.6 us (3.8 at least)
+// in the trace, as without the pass; 512 blocks cost a C2 step 1.8 us, so bf16 steps, which list few rows,
+// launch 32. The pass itself is 1.5 us slower (64.8 -> 66.3) for the 128-bit path's registers beside it.
 __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
     __shared__ union {
         T2Smem t2;
@@ -1153,8 +1155,8 @@ __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2(Params P) {
 }
 
 // force_tier2: every row straight to the 128-bit path, over EA_T2_BLOCKS blocks. A kernel of its own:
-// beside the double-double pass the body spills 413 SGPRs instead of 179 (32 rows of 32K keys 8.9 ms
-// against 6.9).
+// beside the double-double pass the body spills 324 SGPRs instead of 176 (32 rows of 32K keys, that pass
+// included, 6.4 ms against 6.0).
 __global__ void __launch_bounds__(EA_T2_THREADS) ea_tier2_wide(Params P) {
     __shared__ T2Smem S;
     __shared__ int s_last;
@@ -1359,9 +1361,12 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // d = dv = 128: from 3 rows per segment on, up to where the int8 prefill kernel starts. With 1 or 2
 // rows ea_decode (whose 2-row blocks read at the rate of a large copy) takes the steps of 4096 or more
 // segment tiles, and this kernel, with half its tile latency (1.9 against 3.5 us) and splits down to
-// a tile, the shorter ones. 16/8 heads, graph replays of the step, ea_decode -> here: 1 x 600 keys 34.1
-// -> 16.2 us, 1 x 4K 35.1 -> 26.4, 1 x 16K 51.2 -> 38.6, 2 x 15000 66.7 -> 47.9, 16 x 1000 53.1 -> 38.6;
-// the step's kernels 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134, 32 x 4K 117 -> 131. Any other
+// a tile, the shorter ones. 16/8 heads, graph replays of the step, ea_decode -> here: 1 x 600 keys 37.6
+// -> 21.0 us, 1 x 4K 39.5 -> 30.3, 1 x 16K 54.8 -> 42.7, 2 x 15000 68.7 -> 51.3, 16 x 1000 57.1 -> 37.3,
+// 8 x 4000 (4032 tiles) 66.8 -> 47.4;
+// the step's kernels 8 x 4K (4096 tiles) 54.6 -> 53.0, 8 x 16K 120 -> 134, 32 x 4K 117 -> 131. With 8/8
+// heads, 1 row per segment, the line holds too (of 254 decode geometries on either side of it none is slower than
+// on ea_decode by 3%). Any other
 // head size: always (ea_split takes what the pointers or pages do not allow).
 int mrow_rows(const ea_geometry* g, const ea_options* o, int r_seg) {
     if (o->timers || o->kernel == EA_KERNEL_GENERAL) return 0;

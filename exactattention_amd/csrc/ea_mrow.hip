@@ -1,7 +1,7 @@
 // Tier-1 split kernel on the fp64 matrix instructions (gfx950): 4, 8 or 16 query rows of one
-// (sequence, KV head) share every K and V element a wave loads. It takes the steps whose segments
+// (sequence, KV head) share every K and V element a wave loads. It takes the d = 128 steps whose segments
 // have 3 or more rows and too few for the int8 prefill kernel (wide GQA groups, draft chains and
-// trees), and every head size the d = 128 kernels do not cover.
+// trees) or 1 or 2 rows of few keys, and every other head size.
 //
 // What bounds it: on gfx950 an fp64 MFMA runs on the vector unit's own fp64 lanes (measured: 16
 // MACs per cycle and SIMD for v_mfma_f64_16x16x4 (64 cycles), v_mfma_f64_4x4x4 (17 cycles) and
@@ -22,7 +22,8 @@
 // registers spilled the loop's.
 //
 // Rounding: both instructions accumulate as a chain of four single-rounding FMAs in ascending k
-// order (checked bit for bit on the device against fma() chains), so the bounds are those of
+// order (ea_hip_kat_mfma_f64 runs them on given operands, and its test compares them bit for bit with
+// fma()), so the bounds are those of
 // ea_decode's FMA chains: scores 66 u |q|_1 |k|_inf over at most 64 terms per chain, P.V sums of
 // 16 keys per 64-key tile and wave.
 //

@@ -1305,10 +1305,15 @@ int ea::ea_prefill_eligible(const ea_geometry& g, int grp, int kernel, int* ntil
     // once per 1-2 rows in the decode kernel (C4: 0.82 ms here, 2.57 ms there with 4-row blocks)
     // Segments of 24-31 rows (verification of 12-15 draft tokens at GQA 2) come here too when
     // there is enough work: measured on MI355X against the decode kernel (2-row blocks, a
-    // segment's row blocks on one XCD; contiguous K/V, graph replays), the int8 kernel is 14-45%
+    // segment's row blocks on one XCD; contiguous K/V, graph replays), which took the other steps
+    // then, the int8 kernel is 14-45%
     // faster at 24 rows with 8K+ keys on 16+ segments or 32K+ keys on any; at 16 rows the decode
     // kernel is as fast or faster everywhere measured (up to 1.9x at 2K keys, within 3% at 64
-    // segments of 32K keys).
+    // segments of 32K keys). The multi-row kernel takes the steps left now: of 12 to 20 rows, 2K to
+    // 32K keys and 8 to 256 segments all are slower here when K and V are sliced in the step (20 rows,
+    // 256 segments of 8K keys 1362 against 797 us); with the tiles cached 12 to 16 rows are even (within
+    // 10%) on 32 segments of 8K keys and more, and 20 rows faster here from 32K keys on 8 segments, 8K on 32
+    // or 2K on 128 on (448 against 797). The line at 24 rows has not been drawn again.
     const int64_t nseg = (int64_t)g.num_seqs * g.num_kv_heads;
     const bool mid = r_seg >= 24 && g.max_seq_len >= 8192 && (nseg >= 16 || g.max_seq_len >= 32768);
     if (!force && g.num_tokens < 64 && r_seg < PF_RPB && !mid) return 0;
