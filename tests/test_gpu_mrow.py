@@ -221,3 +221,29 @@ def test_matrix_instructions_are_fma_chains(gpu, kind):
                 w4[w, 16 * x + col] = s
     assert np.array_equal(o16.cpu().numpy().view(np.uint64), w16.view(np.uint64))
     assert np.array_equal(o4.cpu().numpy().view(np.uint64), w4.view(np.uint64))
+
+
+@pytest.mark.parametrize("page", [8, 16])
+def test_merge_order_where_another_kernel_stands_in(gpu, page):
+    """A merge order of the reported length on pages the multi-row kernel cannot read: the kernel that
+    stands in merges 64 splits instead of 32 and leaves the order alone. Same bits either way."""
+    rng = np.random.default_rng(31)
+    q, k, v = bf16(rng, (1, 1, 4, 64)), bf16(rng, (1, 1, 16384, 64), "outlier"), bf16(rng, (1, 1, 16384, 64))
+    prob = problem.to_paged(problem.contiguous(q, k, v, [[16000]]), page, rng)
+    ab = default_alpha_bits(64)
+    want, _ = _oracle(prob, ab)
+    got, flags, st = _run(prob, ab, merge_order=list(range(31, -1, -1)))
+    assert st["nsplit"] == 32 and st["mrow_kernel_rows"] == (flags.size if page == 16 else 0), st
+    assert not flags.any() and np.array_equal(got, want), st
+
+
+def test_step_near_the_allocation_free_limit(gpu):
+    """58,000 units whose equal-share plan would not fit where the general kernel's arrays do: uniform
+    splits, many rounds of blocks, within the limit."""
+    from exactattention_amd.hip import workspace_size
+    rng = np.random.default_rng(32)
+    B, Hkv, S = 7250, 8, 8
+    prob = _rand_problem(rng, "normal", "normal", B=B, T=1, Hq=Hkv, Hkv=Hkv, S=S, d=8, dv=96)
+    assert workspace_size(prob["geom"])[0] <= 128 << 20
+    st = _check(prob, default_alpha_bits(8))
+    assert st["decode_equal_share_steps"] == 0, st

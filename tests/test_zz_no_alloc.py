@@ -88,6 +88,16 @@ def test_noalloc_on_the_prefill_and_general_kernels(gpu):
     _both_entry_points(problem.contiguous(q, k, v, np.full((4, 1), 900)), default_alpha_bits(64))
 
 
+def test_noalloc_prefill_of_64_dim_heads(gpu):
+    """Causal prefill of 2048 tokens, 32/8 heads of 64 dims, on the multi-row kernel: 105 MiB of the array."""
+    rng = np.random.default_rng(127)
+    T, Hq, Hkv, d = 2048, 32, 8, 64
+    q, k, v = bf16(rng, (1, T, Hq, d)), bf16(rng, (1, Hkv, T, d)), bf16(rng, (1, Hkv, T, d))
+    dp = _both_entry_points(problem.contiguous(q, k, v, 1 + np.arange(T).reshape(1, T)), default_alpha_bits(d),
+                            expect_kernel="mrow_kernel_rows")
+    assert dp.ws_bytes > (100 << 20), dp.ws_bytes
+
+
 def test_noalloc_long_context_workspace(gpu):
     """16 ragged sequences planned for 131,072 keys (the long-context bound: 64 KV splits, about
     72 MB of the array's 128 MiB); only the actual lengths are read."""
